@@ -3,11 +3,11 @@
 // trinix_attn_bwd validates the arguments, computes delta = rowsum(dO * O)
 // into the caller's workspace and launches the dK/dV and dQ kernels: the
 // bf16/fp16 MFMA pipeline (attn_bwd16.h, instantiated per (dtype, head_dim)
-// in attn_bwd16_*.hip) for head_dim 64/128, dropout included, the generic
-// fp32-product kernels (attn_bwd_generic.hip) for fp32 and head_dim 256.
+// in attn_bwd16_*.hip) for head_dim 64/128, the kernels whose P and dZ keep
+// fp32 precision (attn_bwd_generic.h, attn_bwd_generic_*.hip) for fp32 and head_dim 256.
 #include <cstdint>
 
-#include "attn_bwd16.h"
+#include "attn_bwd_generic.h"
 #include "host_plan.h"
 
 namespace trinix {
@@ -42,6 +42,42 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const uint16_t* __restri
   // dmul = 1 - p with dropout: the kernels then use keep*dP - delta*(1-p)
   // and apply 1/(1-p) to dq and dk in their epilogues
   if (t == 0 && row < rows) delta[row] = lse[row] == -INFINITY ? 0.f : acc * dmul;
+}
+
+// The same for fp32 rows (any 4-byte aligned start): D/4 lanes per row.
+template <int D>
+__global__ __launch_bounds__(256) void bwd_delta_f32(const float* __restrict__ o, int64_t o_sb, int64_t o_ss,
+                                                     int64_t o_sh, const float* __restrict__ dout, int64_t do_sb,
+                                                     int64_t do_ss, int64_t do_sh, const float* __restrict__ lse,
+                                                     float* __restrict__ delta, float dmul, int Hq, int Sq,
+                                                     int64_t rows) {
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int LPR = D / 4, RPB = 256 / LPR;
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  const int t = threadIdx.x % LPR;
+  float acc = 0.f;
+  if (row < rows) {
+    const int i = (int)(row % Sq);
+    const int64_t bh = row / Sq;
+    const int h = (int)(bh % Hq);
+    const int64_t b = bh / Hq;
+    const f32x4_t ov = *(const f32x4_any*)(o + b * o_sb + i * o_ss + h * o_sh + t * 4);
+    const f32x4_t dv = *(const f32x4_any*)(dout + b * do_sb + i * do_ss + h * do_sh + t * 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc += ov[e] * dv[e];
+  }
+#pragma unroll
+  for (int m = LPR / 2; m >= 1; m /= 2) acc += __shfl_xor(acc, m);
+  if (t == 0 && row < rows) delta[row] = lse[row] == -INFINITY ? 0.f : acc * dmul;
+}
+
+template <int D>
+hipError_t launch_delta_f32(const BwdParams& p, hipStream_t st) {
+  constexpr int RPB = 256 / (D / 4);
+  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
+  return launch_kernel(&bwd_delta_f32<D>, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st,
+                       (const float*)p.o, p.o_sb, p.o_ss, p.o_sh, (const float*)p.dout, p.do_sb, p.do_ss, p.do_sh,
+                       p.lse, p.delta, p.use_dropout ? 1.f / p.drop_scale : 1.f, p.Hq, p.Sq, rows);
 }
 
 template <class E, int D>
@@ -128,13 +164,19 @@ extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) {
 
   hipStream_t st = (hipStream_t)stream;
   hipError_t err;
-  if (a->dtype == TRINIX_F32 || a->head_dim == 256) {
-    if (!bwd_generic_fits(p)) return TRINIX_ERR_BAD_SHAPE;
-    err = launch_bwd_generic(p, a->dtype, (int)a->head_dim, st);
+  if (a->dtype == TRINIX_F32) {
+    p.rows16 = rows_aligned16(a->q, a->q_stride) && rows_aligned16(a->k, a->k_stride) &&
+               rows_aligned16(a->v, a->v_stride) && rows_aligned16(a->dout, a->dout_stride);
+    const int D = (int)a->head_dim;
+    err = D == 64 ? launch_delta_f32<64>(p, st) : D == 128 ? launch_delta_f32<128>(p, st) : launch_delta_f32<256>(p, st);
+    if (err == hipSuccess) err = launch_bwd_generic_f32(p, D, plan, st);
     return err == hipSuccess ? TRINIX_OK : TRINIX_ERR_LAUNCH;
   }
   const bool bf = a->dtype == TRINIX_BF16;
-  if (a->head_dim == 128) {
+  if (a->head_dim == 256) {
+    err = bf ? launch_delta<BF16, 256>(p, st) : launch_delta<F16, 256>(p, st);
+    if (err == hipSuccess) err = bf ? launch_bwd_generic_bf16(p, plan, st) : launch_bwd_generic_f16(p, plan, st);
+  } else if (a->head_dim == 128) {
     err = bf ? launch_delta<BF16, 128>(p, st) : launch_delta<F16, 128>(p, st);
     if (err == hipSuccess) err = bf ? launch_bwd16_bf16_d128(p, feat, st) : launch_bwd16_f16_d128(p, feat, st);
   } else {

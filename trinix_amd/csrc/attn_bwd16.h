@@ -68,31 +68,7 @@ struct BwdParams {
   const uint64_t* drop_state;  // {seed, offset} in device memory, read in place of the four above; or null
   const uint32_t* keep_map;    // the forward's keep bits (index_map.h), read in place of Philox; or null
   int64_t km_nbi, km_nbj;      // its row / key blocks per (batch, q-head)
-};
-
-// Allowed (i, j): j - i in [dlo, dhi] (causal: j <= i; window: -wl <= j-i <= wr).
-struct Band {
-  int dlo, dhi;
-  __device__ Band(const BwdParams& p) { band_offsets(p.causal != 0, p.has_window != 0, p.wl, p.wr, dlo, dhi); }
-  __device__ bool ok(int i, int j) const { return j - i >= dlo && j - i <= dhi; }
-};
-
-// Allowed range [lo, lo + span] of one index as an unsigned interval test:
-// (uint32_t)(x - lo) <= span is one subtract and one compare per element (an
-// empty range gets lo = INT_MAX, which no x in [0, 2^30) passes).
-struct Span {
-  int lo;
-  uint32_t span;
-  __device__ Span(int64_t a, int64_t b) {
-    if (b < a) {
-      lo = INT_MAX;
-      span = 0u;
-    } else {
-      lo = (int)a;
-      span = (uint32_t)(b - a);
-    }
-  }
-  __device__ bool ok(int x) const { return (uint32_t)(x - lo) <= span; }
+  int rows16;                  // fp32: q, k, v and dout take 16-byte copies (rows_aligned16)
 };
 
 // LDS operand reads of a row-major, D-wide 16-bit tile swizzled with
@@ -1010,12 +986,5 @@ hipError_t launch_bwd16_bf16_d64(const BwdParams& p, int feat, hipStream_t st);
 hipError_t launch_bwd16_bf16_d128(const BwdParams& p, int feat, hipStream_t st);
 hipError_t launch_bwd16_f16_d64(const BwdParams& p, int feat, hipStream_t st);
 hipError_t launch_bwd16_f16_d128(const BwdParams& p, int feat, hipStream_t st);
-
-// The generic backward (attn_bwd_generic.hip): fp32 products, any dtype
-// (TRINIX_F32 / F16 / BF16), head_dim 64, 128 or 256, dropout, ALiBi and
-// mask read per element.  Launches its own delta pre-pass.
-hipError_t launch_bwd_generic(const BwdParams& p, int dtype, int D, hipStream_t st);
-// Whether the generic kernels' grids fit 2^31 workgroups.
-bool bwd_generic_fits(const BwdParams& p);
 
 }  // namespace trinix

@@ -1,6 +1,8 @@
 // Launch parameters of the attention kernels and the small device helpers
 // they share (mask element loads, dropout, cross-lane reductions).
 #pragma once
+#include <climits>
+
 #include "common.h"
 #include "host_plan.h"
 #include "trinix_attn.h"
@@ -43,6 +45,7 @@ struct FwdParams {
   uint16_t* qn_out;  // the normalised q, contiguous (B, Sq, Hq, D), or null
   uint32_t* keep_map;    // dropout keep bits written for the backward (index_map.h), or null
   int64_t km_nbi, km_nbj;  // its row / key blocks per (batch, q-head)
+  int rows16;              // fp32: k and v take 16-byte copies (rows_aligned16)
   // work items of the per-item key split (Cfg16 ks = 0), longest chain
   // first: row block << 2 | split << 1 | half (plan_split_rows)
   uint8_t row_items[kMaxRowItems];
@@ -144,6 +147,32 @@ __device__ inline uint32_t keep_word(uint32_t m, int v) {
   return (uint32_t)w;
 }
 
+// Allowed (i, j): j - i in [dlo, dhi] (causal: j <= i; window: -wl <= j-i <= wr).
+struct Band {
+  int dlo, dhi;
+  template <class P>
+  __device__ explicit Band(const P& p) { band_offsets(p.causal != 0, p.has_window != 0, p.wl, p.wr, dlo, dhi); }
+  __device__ bool ok(int i, int j) const { return j - i >= dlo && j - i <= dhi; }
+};
+
+// Allowed range [lo, lo + span] of one index as an unsigned interval test:
+// (uint32_t)(x - lo) <= span is one subtract and one compare per element (an
+// empty range gets lo = INT_MAX, which no x in [0, 2^30) passes).
+struct Span {
+  int lo;
+  uint32_t span;
+  __device__ Span(int64_t a, int64_t b) {
+    if (b < a) {
+      lo = INT_MAX;
+      span = 0u;
+    } else {
+      lo = (int)a;
+      span = (uint32_t)(b - a);
+    }
+  }
+  __device__ bool ok(int x) const { return (uint32_t)(x - lo) <= span; }
+};
+
 // Combine a value with the one held by lane l ^ 32 (v_permlane32_swap).
 __device__ inline float xlane_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -165,6 +194,14 @@ hipError_t launch_attn16_f16_d64(const FwdParams& p, Cfg16 cfg, int feat, hipStr
 hipError_t launch_attn16_f16_d128(const FwdParams& p, Cfg16 cfg, int feat, hipStream_t st);
 hipError_t launch_attn16_bf16_d256(const FwdParams& p, Cfg16 cfg, int feat, hipStream_t st);
 hipError_t launch_attn16_f16_d256(const FwdParams& p, Cfg16 cfg, int feat, hipStream_t st);
+// The fp32 kernel with ks wavefronts per 32 query rows (attn_fwd_f32.hip).
+hipError_t launch_attn_f32(const FwdParams& p, int head_dim, int ks, hipStream_t st);
+
+// fp32 rows that 16-byte copies can read, 32 of them within 32-bit offsets
+inline bool rows_aligned16(const void* ptr, const int64_t st[4]) {
+  return ((uintptr_t)ptr & 15) == 0 && st[0] % 4 == 0 && st[1] % 4 == 0 && st[2] % 4 == 0 && st[1] >= 0 &&
+         st[1] < (1ll << 24);
+}
 
 
 // Feature bits of a launch (compile-time flags of the 16-bit kernels).

@@ -241,6 +241,22 @@ int64_t clamp_window(int64_t w) {
   return w < -lim ? -lim : (w > lim ? lim : w);
 }
 
+// Two wavefronts per 32 keys or rows (half the chain of tiles, twice the
+// workgroups, but twice the tile copies per product and a merge through LDS)
+// in the fp32 and head_dim 256 kernels, where `wgs` workgroups of one
+// wavefront per 32 would leave the chip with few rounds.  Measured (forward +
+// backward, us, one | two wavefronts):
+//   dK/dV  fp32 D=64 384 workgroups 402 | 344, 1024: 1435 | 1410; D=128 288:
+//          430 | 379, 512: 1448 | 1468; D=256 bf16 256: 432 | 344, 4096: 4030 |
+//          4430, fp16 256: 502 | 400, 512: 395 | 421
+//   dQ     fp32 D=64 384: 408 | 344, 1024: 1519 | 1410; D=128 288: 398 | 379,
+//          512: 1670 | 1468; D=256 bf16 256: 367 | 344, 2048: 4030 | 4300, fp16
+//          512: 395 | 423
+//   forward (fp32) D=64 384: 111 | 79, 1024: 325 | 313; D=128 512: 331 | 353
+static bool two_per_group(int64_t head_dim, int64_t wgs, int64_t limit128) {
+  return wgs <= (head_dim == 64 ? 4096 : head_dim == 128 ? limit128 : 384);
+}
+
 int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   const bool f32 = a->dtype == TRINIX_F32;
   const bool plain = !a->mask && !(a->dropout_p > 0.f);
@@ -250,6 +266,12 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   if (a->q_norm_weight) cfg.ks = 1;  // the fused q RMSNorm is built without the key split
   pl->n_items = 0;
   pl->num_mblk = 0;
+  pl->f32_ks = 1;
+  if (f32 && a->head_dim <= 128) {
+    pl->f32_ks = two_per_group(a->head_dim, a->batch * a->nheads_q * ((a->seqlen_q + 127) / 128), 384) ? 2 : 1;
+    if (const char* env = getenv("TRINIX_F32_KS"))  // tuning and tests
+      if (env[0] == '1' || env[0] == '2') pl->f32_ks = env[0] - '0';
+  }
   if (cfg.ks == 0) {  // per-item key split: the item table, or no split
     const int n = split_ok ? plan_split_rows(a->seqlen_q, a->seqlen_k, a->batch * a->nheads_q, 32 * cfg.nw, cfg.bn,
                                              pl->row_items, kMaxRowItems) : 0;
@@ -261,7 +283,7 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
     }
   }
   if (f32 || cfg.ks != 0) {
-    const int bm = f32 ? 32 * kWavesF32 : 32 * cfg.nw / cfg.ks;
+    const int bm = f32 ? 32 * kWavesF32 / pl->f32_ks : 32 * cfg.nw / cfg.ks;
     pl->num_mblk = (int)((a->seqlen_q + bm - 1) / bm);
   }
   pl->cfg = cfg;
@@ -271,11 +293,34 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
 }
 
 int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl) {
-  pl->num_kblk = (int)((a->seqlen_k + 127) / 128);
-  pl->dq_wide = a->dtype != TRINIX_F32 && pick_dq_wide(a->head_dim, a->batch, a->nheads_q, a->seqlen_q,
-                                                       a->causal || a->has_window, a->mask != nullptr);
-  pl->num_mblk = (int)((a->seqlen_q + (pl->dq_wide ? 255 : 127)) / (pl->dq_wide ? 256 : 128));
-  if (a->batch * a->nheads_q * pl->num_mblk >= (1ll << 31) || a->batch * a->nheads_kv * pl->num_kblk >= (1ll << 31))
+  const bool f32 = a->dtype == TRINIX_F32;
+  const int64_t D = a->head_dim;
+  pl->generic = f32 || D == 256;
+  pl->dq_wide = !pl->generic && pick_dq_wide(D, a->batch, a->nheads_q, a->seqlen_q, a->causal || a->has_window,
+                                             a->mask != nullptr);
+  pl->dq_ks = pl->kv_ks = pl->dq_hs = pl->kv_hs = 1;
+  if (pl->generic) {
+    if (D == 256) {  // column splits: the kernels' registers
+      pl->kv_hs = f32 ? 4 : 2;
+      pl->dq_hs = a->dtype == TRINIX_BF16 ? 1 : 2;
+    }
+    if (!(f32 && D == 256)) {  // (whose tiles fill the LDS)
+      pl->kv_ks = two_per_group(D, a->batch * a->nheads_kv * ((a->seqlen_k + 127) / 128) * pl->kv_hs, 384) ? 2 : 1;
+      pl->dq_ks = two_per_group(D, a->batch * a->nheads_q * ((a->seqlen_q + 127) / 128) * pl->dq_hs, 1024) ? 2 : 1;
+      if (const char* env = getenv("TRINIX_BWD_GENERIC")) {  // "dq_ks,kv_ks" (tuning and tests)
+        int ks = 0, kks = 0;
+        if (sscanf(env, "%d,%d", &ks, &kks) == 2 && (ks == 1 || ks == 2) && (kks == 1 || kks == 2)) {
+          pl->dq_ks = ks;
+          pl->kv_ks = kks;
+        }
+      }
+    }
+  }
+  const int bm = pl->dq_wide ? 256 : 128 / pl->dq_ks, bk = 128 / pl->kv_ks;
+  pl->num_kblk = (int)((a->seqlen_k + bk - 1) / bk);
+  pl->num_mblk = (int)((a->seqlen_q + bm - 1) / bm);
+  if (a->batch * a->nheads_q * pl->num_mblk * pl->dq_hs >= (1ll << 31) ||
+      a->batch * a->nheads_kv * pl->num_kblk * pl->kv_hs >= (1ll << 31))
     return TRINIX_ERR_BAD_SHAPE;
   return TRINIX_OK;
 }

@@ -59,6 +59,7 @@ struct FwdPlan {
   Cfg16 cfg;           // 16-bit kernels; cfg.ks = 0 only with n_items > 0
   int num_mblk;        // work items per (batch, q-head)
   int64_t total_work;  // workgroups
+  int f32_ks;          // fp32: wavefronts per 32 rows (row blocks of 128 / f32_ks)
   int n_items;         // entries of row_items (cfg.ks == 0)
   uint8_t row_items[kMaxRowItems];
 };
@@ -66,11 +67,15 @@ struct FwdPlan {
 // workgroups.  For validated arguments.
 int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl);
 
-// Launch plan of trinix_attn_bwd's 16-bit kernels: 128-key blocks (dK/dV)
-// and 128- or 256-row blocks (dQ).
+// Launch plan of trinix_attn_bwd: 128-key blocks (dK/dV) and 128- or 256-row
+// blocks (dQ).  `generic` (fp32, and 16-bit at head_dim 256:
+// attn_bwd_generic.h): blocks of 128 / kv_ks keys and 128 / dq_ks rows, their
+// columns over kv_hs and dq_hs workgroups.
 struct BwdPlan {
   int num_kblk, num_mblk;
   bool dq_wide;
+  bool generic;
+  int dq_ks, kv_ks, dq_hs, kv_hs;
 };
 int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl);
 

@@ -31,6 +31,14 @@ __device__ inline void dma_4b_s(uint32_t offset, uint64_t base, uint32_t lds_bas
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "memory", "m0");
 }
 
+// The same two copies from a per-lane 64-bit address (any row stride).
+__device__ inline void dma_16b(const void* src, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_base) : "memory", "m0");
+}
+__device__ inline void dma_4b(const void* src, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds_base) : "memory", "m0");
+}
+
 // Wave-uniform copy of a pointer as a 64-bit SGPR value.
 __device__ inline uint64_t uniform_ptr(const void* ptr) {
   const uint64_t x = (uint64_t)(uintptr_t)ptr;
