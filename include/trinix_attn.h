@@ -372,6 +372,16 @@ typedef struct trinix_attn_bwd_args {
   const void* dropout_keep_map;
 } trinix_attn_bwd_args;
 int trinix_attn_bwd(const trinix_attn_bwd_args* args, void* stream);
+/* The same with workspace for partial sums: where whole 128-key blocks would
+ * leave the GPU partly idle (few KV heads, short sequences), dk and dv are
+ * summed from pieces of them.  trinix_attn_bwd_workspace gives the bytes the
+ * call needs (0: none, trinix_attn_bwd does the same work);
+ * trinix_attn_bwd_ws takes at least that many, 16-byte aligned
+ * (TRINIX_ERR_BAD_ARGUMENT otherwise), free for reuse by later work on the
+ * stream.  Deterministic, like trinix_attn_bwd, whose results differ from it
+ * by the order of fp32 sums only. */
+int trinix_attn_bwd_workspace(const trinix_attn_bwd_args* args, int64_t* workspace_bytes);
+int trinix_attn_bwd_ws(const trinix_attn_bwd_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ALiBi bias, reference trinix/kernels/alibi_kernel.py:8-54:
  *   out[h*out_stride_h + i*out_stride_i + j] = -slopes[h*slope_stride] * |i - j|

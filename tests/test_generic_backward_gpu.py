@@ -8,8 +8,9 @@ Bars against float64 autograd of the oracle.  Elementwise the repository's
 (twice the eager error of the dtype plus 2e-3, or for fp32 1e-5, of the
 scale).  In the 2-norm, 16-bit: the inputs' products are exact and P and dZ
 carry 16 or more bits, so what is left is the rounding of each gradient and of
-the saved output (through delta): at most a unit roundoff each, together 2u of
-the gradient's norm (P or dZ rounded to 16 bits would pass that)."""
+the saved output (through delta), uniform within u of an element: u / sqrt(3)
+of the norm each, 0.82 u together; the bar is u (P and dZ rounded to 16 bits
+show 1.2 u)."""
 import pytest
 import torch
 
@@ -44,7 +45,7 @@ def _compare(hip, ts, do, dtype, **kw):
         scale, err_h, err_e = t.abs().max().item(), (h - t).abs().max().item(), (e - t).abs().max().item()
         assert err_h <= 2 * err_e + (1e-5 if dtype == torch.float32 else 2e-3) * scale, (name, err_h, err_e, scale)
         if dtype in UNIT and name != "out":
-            assert (h - t).norm() <= 2 * UNIT[dtype] * t.norm() + 1e-12, (name, (h - t).norm() / t.norm())
+            assert (h - t).norm() <= UNIT[dtype] * t.norm(), (name, (h - t).norm() / t.norm())
 
 
 @pytest.mark.parametrize("ks", ["1", "2"])
@@ -99,4 +100,4 @@ def test_fp16_head_dim_256_gradient_range(exponent):
     truth = _grads(orc.functional_attention, [t.double() for t in ts], do.double(), causal=True)
     for name, h, t in list(zip(("out", "dq", "dk", "dv"), hip, truth))[1:]:
         err = (h.cpu().double() - t).norm()
-        assert err <= 2 * UNIT[torch.float16] * t.norm() + 2.0 ** -24 * t.numel() ** 0.5, (name, (err / t.norm()).item())
+        assert err <= UNIT[torch.float16] * t.norm() + 2.0 ** -24 * t.numel() ** 0.5, (name, (err / t.norm()).item())

@@ -169,6 +169,8 @@ SIGNATURES = {
     "trinix_attn_fwd_splitkv": (c_int32, [POINTER(AttnFwdArgs), c_void_p, c_int64, c_void_p]),
     "trinix_attn_fwd_splitkv_noalloc": (c_int32, [POINTER(AttnFwdArgs), c_void_p]),
     "trinix_attn_bwd": (c_int32, [POINTER(AttnBwdArgs), c_void_p]),
+    "trinix_attn_bwd_workspace": (c_int32, [POINTER(AttnBwdArgs), POINTER(c_int64)]),
+    "trinix_attn_bwd_ws": (c_int32, [POINTER(AttnBwdArgs), c_void_p, c_int64, c_void_p]),
     "trinix_qk_norm": (
         c_int32,
         [c_void_p, POINTER(c_int64), c_void_p, POINTER(c_int64), c_int64, c_int64, c_int64, c_int64, c_int32,

@@ -94,7 +94,9 @@ hipError_t launch_delta(const BwdParams& p, hipStream_t st) {
 
 using namespace trinix;
 
-extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) {
+namespace {
+
+int run_bwd(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_bytes, bool split, void* stream) {
   const int vrc = validate_bwd_args(a);
   if (vrc != TRINIX_OK) return vrc;
 
@@ -140,8 +142,13 @@ extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) {
   p.bm_sh = a->blockmap_stride[1];
   p.bm_cols = (int)((a->seqlen_k + 63) / 64);
   BwdPlan plan;
-  const int prc = plan_bwd(a, &plan);
+  const int prc = plan_bwd(a, &plan, split);
   if (prc != TRINIX_OK) return prc;
+  if (plan.ws_bytes > 0 && (!workspace || workspace_bytes < plan.ws_bytes || ((uintptr_t)workspace & 15) != 0))
+    return TRINIX_ERR_BAD_ARGUMENT;
+  p.kv_T = plan.kv_T;
+  p.kv_P = plan.kv_P;
+  p.part = (float*)workspace;
   p.num_kblk = plan.num_kblk;
   p.num_mblk = plan.num_mblk;
   p.dq_wide = plan.dq_wide ? 1 : 0;
@@ -184,4 +191,23 @@ extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) {
     if (err == hipSuccess) err = bf ? launch_bwd16_bf16_d64(p, feat, st) : launch_bwd16_f16_d64(p, feat, st);
   }
   return err == hipSuccess ? TRINIX_OK : TRINIX_ERR_LAUNCH;
+}
+
+}  // namespace
+
+extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) { return run_bwd(a, nullptr, 0, false, stream); }
+
+extern "C" int trinix_attn_bwd_workspace(const trinix_attn_bwd_args* a, int64_t* bytes) {
+  if (!bytes) return TRINIX_ERR_NULL_POINTER;
+  *bytes = 0;
+  const int vrc = validate_bwd_args(a);
+  if (vrc != TRINIX_OK) return vrc;
+  BwdPlan plan;
+  const int prc = plan_bwd(a, &plan, true);
+  if (prc == TRINIX_OK) *bytes = plan.ws_bytes;
+  return prc;
+}
+
+extern "C" int trinix_attn_bwd_ws(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
+  return run_bwd(a, workspace, workspace_bytes, true, stream);
 }

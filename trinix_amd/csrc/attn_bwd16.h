@@ -68,6 +68,10 @@ struct BwdParams {
   const uint64_t* drop_state;  // {seed, offset} in device memory, read in place of the four above; or null
   const uint32_t* keep_map;    // the forward's keep bits (index_map.h), read in place of Philox; or null
   int64_t km_nbi, km_nbj;      // its row / key blocks per (batch, q-head)
+  // dK/dV in pieces of at most kv_T items (0: whole key blocks), kv_P per
+  // (batch, KV head); fp32 partials of the key blocks of several pieces
+  int kv_T, kv_P;
+  float* part;
   int rows16;                  // fp32: q, k, v and dout take 16-byte copies (rows_aligned16)
 };
 
@@ -229,7 +233,61 @@ __device__ inline uint32_t transpose_keep_block(uint32_t a, int lane) {
 // (1-p)), the delta kernel having scaled delta = rowsum(dO*O) by 1-p.  The
 // 1/(1-p) of Pd = keep P/(1-p) and of dZ = P (keep dP/(1-p) - delta) =
 // dZ'/(1-p) is applied once per output element in the epilogue.
+//
+// With p.kv_T the items of a key block are cut into pieces (plan_bwd_pieces),
+// each a workgroup; a block of several pieces leaves fp32 partial sums that
+// bwd_dkdv_reduce adds in order (no atomics: bitwise the same every run).
+// Measured, forward + backward, bf16 causal D = 128, us, whole | pieces: B=2
+// S=2048 16/4 heads 342 | 214 (dK/dV had 128 workgroups, the longest with 128
+// items), S=2400 16/4 382 | 190, S=1000 32/8 179 | 128, S=4100 32/8 805 | 700,
+// S=8192 16/4 1612 | 1377; where the plan keeps whole blocks: S=4000 16/16 365 |
+// 375, S=8192 32/8 2250 | 2354.
 // ---------------------------------------------------------------------------
+// Key block and piece of it (np, pk) of the `index`-th piece of a group: lane k
+// counts the pieces of key block k (num_kblk <= 64), a prefix sum finds it.
+__device__ inline int lane_piece_ends(const BwdParams& p, const Band& band, int lane) {
+  int n = lane < p.num_kblk ? bwd_pieces(bwd_kv_items(lane, 128, p.G, p.Sq, p.Sk, band.dlo, band.dhi, 64), p.kv_T) : 0;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    const int o = __shfl_up(n, m);
+    if (lane >= m) n += o;
+  }
+  return n;
+}
+__device__ inline int piece_block(const BwdParams& p, const Band& band, int lane, int index, int& np, int& pk) {
+  const int end = lane_piece_ends(p, band, lane);
+  const int kblk = min((int)__popcll(__builtin_amdgcn_ballot_w64(end <= index)), p.num_kblk - 1);
+  const int hi = __builtin_amdgcn_readlane(end, kblk), lo = kblk ? __builtin_amdgcn_readlane(end, kblk - 1) : 0;
+  np = hi - lo;
+  pk = index - lo;
+  return kblk;
+}
+
+// Sums the partials of the key blocks of several pieces: a thread adds four
+// head_dim elements of one key of dV (blockIdx.y = 0) or dK (1) over the
+// pieces, in order.
+template <class E, int D, bool DROP>
+__global__ __launch_bounds__(256) void bwd_dkdv_reduce(const BwdParams p) {
+  constexpr int BK = 128, DB = D / 32, SLICES = 4 * DB * 4 * 64 / 256;
+  const int tid = threadIdx.x, lane = tid & 63, sb = blockIdx.y;
+  const int sl = blockIdx.x % SLICES, blk = blockIdx.x / SLICES, kblk = blk % p.num_kblk, group = blk / p.num_kblk;
+  const Band band(p);
+  const int end = lane_piece_ends(p, band, lane);
+  const int hi = __builtin_amdgcn_readlane(end, kblk), lo = kblk ? __builtin_amdgcn_readlane(end, kblk - 1) : 0;
+  if (hi - lo < 2) return;  // written by its only piece
+  const int unit = sl * 256 + tid, kg = unit / (DB * 4 * 64), dq = unit / 64 % (DB * 4), l = unit & 63;
+  const float* part = p.part + (((int64_t)group * p.kv_P + lo) * 2 + sb) * BK * D + unit * 4;
+  f32x4_t s = *(const f32x4_t*)part;
+  for (int k = 1; k < hi - lo; ++k) s += *(const f32x4_t*)(part + (int64_t)k * 2 * BK * D);
+  const int j = kblk * BK + kg * 32 + (l & 31), d0 = dq * 8 + (l >> 5) * 4;
+  if (j >= p.Sk) return;
+  const int b = group / p.Hkv, hkv = group % p.Hkv;
+  uint16_t* row = sb ? p.dk + b * p.dk_sb + hkv * p.dk_sh + (int64_t)j * p.dk_ss
+                     : p.dv + b * p.dv_sb + hkv * p.dv_sh + (int64_t)j * p.dv_ss;
+  const float f = (sb ? p.scale : 1.f) * (DROP ? p.drop_scale : 1.f);
+  *(u32x2_t*)(row + d0) = (u32x2_t){E::pack(s[0] * f, s[1] * f), E::pack(s[2] * f, s[3] * f)};
+}
+
 template <class E, int D, bool ALIBI, bool MASK, int DROP>
 __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
   DropKey dkey{};
@@ -254,13 +312,22 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
   const int kg = wave % NG;
   const int g = lane >> 5;
 
-  const KvItem wi = bwd_kv_item((int)blockIdx.x, p.B, p.Hkv, p.num_kblk, p.causal != 0);  // (index_map.h)
-  const int kblk = wi.kblk, hkv = wi.hkv, b = wi.b;
+  const Band band(p);
+  // (index_map.h) key block, and which of its pieces (one unless kv_T cuts it)
+  int kblk, hkv, b, np = 1, pk = 0, slot = 0;
+  if (p.kv_T == 0) {
+    const KvItem wi = bwd_kv_item((int)blockIdx.x, p.B, p.Hkv, p.num_kblk, p.causal != 0);
+    kblk = wi.kblk, hkv = wi.hkv, b = wi.b;
+  } else {
+    const KvPiece pc = bwd_kv_piece((int)blockIdx.x, p.B * p.Hkv, p.kv_P);
+    b = pc.group / p.Hkv, hkv = pc.group % p.Hkv;
+    slot = pc.group * p.kv_P + pc.index;
+    kblk = piece_block(p, band, lane, pc.index, np, pk);
+  }
   const int kb0 = kblk * BK;
   const int j0 = kb0 + kg * 32;
   const int j = j0 + (lane & 31);
   const int jc = min(j, p.Sk - 1);
-  const Band band(p);
   // queries this lane's key may see: j - dhi <= i <= j - dlo, 0 <= i < Sq (none if j >= Sk)
   const Span qspan = j < p.Sk ? Span(max((int64_t)0, (int64_t)j - band.dhi), min((int64_t)p.Sq - 1, (int64_t)j - band.dlo))
                               : Span(1, 0);
@@ -270,7 +337,10 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
   int qt_lo, qt_hi;
   bwd_query_tiles(kb0, BK, p.Sq, p.Sk, band.dlo, band.dhi, BQ, qt_lo, qt_hi);
   const int nqt = qt_hi - qt_lo;
-  const int n_items = nqt > 0 ? p.G * nqt : 0;  // item = (q-head of the group, query tile)
+  // item = (q-head of the group, query tile); this workgroup's run of them
+  const int all_items = nqt > 0 ? p.G * nqt : 0, it0 = bwd_piece_first(all_items, np, pk);
+  const int n_items = bwd_piece_first(all_items, np, pk + 1) - it0;
+  const int gh0 = nqt > 0 ? it0 / nqt : 0, qt0 = nqt > 0 ? qt_lo + it0 % nqt : qt_lo;
 
   // ---- tile copies: Q and dO rows (16-byte units, swizzled), lse and delta
   auto ld_row = [&](int l) __attribute__((always_inline)) { return tile_copy_row(wave, LPW, l, lane, UPR); };
@@ -584,9 +654,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
-    if (n_items > 0) load_item(Item{0, qt_lo}, I0{});
+    if (n_items > 0) load_item(Item{gh0, qt0}, I0{});
     write_lse();
-    Item ia{0, qt_lo}, ib{0, qt_lo};
+    Item ia{gh0, qt0}, ib{gh0, qt0};
     auto step = [&](auto sa_c, auto pa_c, int s) __attribute__((always_inline)) {
       constexpr int SA = decltype(sa_c)::value, PA = decltype(pa_c)::value;
       __builtin_amdgcn_s_waitcnt(0);  // this wavefront's copies and P writes landed
@@ -611,6 +681,18 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
       if (s + 5 <= n_items) step(I2{}, I1{}, s + 5);
     }
 
+    // ---- epilogue: a piece's fp32 partial sums, in the order of the lanes
+    // (bwd_dkdv_reduce adds them up)
+    if (np > 1) {
+      float* part = p.part + ((int64_t)slot * 2 + (SB ? 1 : 0)) * BK * D + (kg * DB * 4 * 64 + lane) * 4;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int vq = 0; vq < 4; ++vq)
+          *(f32x4_t*)(part + (db * 4 + vq) * 256) =
+              (f32x4_t){acc[db][vq * 4], acc[db][vq * 4 + 1], acc[db][vq * 4 + 2], acc[db][vq * 4 + 3]};
+      return;
+    }
     // ---- epilogue: dV, or dK = scale * dZ^T Q
     if (j < p.Sk) {
       uint16_t* row = SB ? p.dk + b * p.dk_sb + hkv * p.dk_sh + (int64_t)j * p.dk_ss
@@ -942,9 +1024,12 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_bwd_dq(const BwdParams p) {
 // kernels (0 none, 1 regenerated keep mask, 2 the forward's keep map).
 template <class E, int D, bool A, bool M, int DROP>
 hipError_t launch_bwd_pair(const BwdParams& p, hipStream_t st) {
-  const dim3 g_kv((unsigned)(p.B * p.Hkv * p.num_kblk)), g_q((unsigned)(p.B * p.Hq * p.num_mblk)), blk(256),
+  const dim3 g_kv((unsigned)(p.B * p.Hkv * (p.kv_T ? p.kv_P : p.num_kblk))), g_q((unsigned)(p.B * p.Hq * p.num_mblk)), blk(256),
       blk_kv(512);
-  const hipError_t e = launch_kernel(&attn_bwd_dkdv<E, D, A, M, DROP>, g_kv, blk_kv, 0, st, p);
+  hipError_t e = launch_kernel(&attn_bwd_dkdv<E, D, A, M, DROP>, g_kv, blk_kv, 0, st, p);
+  if (e == hipSuccess && p.kv_T)
+    e = launch_kernel(&bwd_dkdv_reduce<E, D, DROP != 0>, dim3((unsigned)(p.B * p.Hkv * p.num_kblk * (D / 32 * 4)), 2), blk, 0,
+                      st, p);
   if (e != hipSuccess) return e;
   if constexpr (D == 128 && !M)
     if (p.dq_wide) return launch_kernel(&attn_bwd_dq<E, D, A, M, DROP, 8, 128>, g_q, blk_kv, 0, st, p);

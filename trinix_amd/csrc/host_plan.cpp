@@ -3,6 +3,12 @@
 // status, a plan or a tile shape.
 #include "host_plan.h"
 
+#ifndef __host__  // plain C++: index_map.h's attributes are empty
+#define __host__
+#define __device__
+#endif
+#include "index_map.h"
+
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -292,7 +298,60 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   return TRINIX_OK;
 }
 
-int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl) {
+// dK/dV of the 16-bit kernels in pieces: where whole key blocks leave the
+// 256 CUs (one workgroup each) with a long chain and idle neighbours -- few
+// (batch, KV head) pairs, a causal band, or a last round nearly empty -- the
+// blocks' items are cut into pieces of at most T that fill one or two rounds.
+// Costs are in items (64 query rows of one q-head; 1.7 us at D = 128, 1.0 at
+// D = 64, two wavefronts per SIMD busy): the longest chain or the share of a
+// CU, against T per round plus the partials' write and read (about 4 TB/s) and
+// one more launch (7 us).  Taken when it saves a tenth (figures beside
+// attn_bwd_dkdv, attn_bwd16.h: forward + backward 342 -> 214 us at B=2 S=2048
+// 16/4 heads; pieces lose 3..30% where whole blocks fill the chip).
+static void plan_bwd_pieces(const trinix_attn_bwd_args* a, BwdPlan* pl) {
+  constexpr int BK = 128, BQ = 64;
+  constexpr int64_t slots = kSmallGrid;
+  const int D = (int)a->head_dim, G = (int)(a->nheads_q / a->nheads_kv), nk = pl->num_kblk;
+  const int64_t groups = a->batch * a->nheads_kv;
+  if (nk > kMaxSplitKblk || groups * nk > 4 * slots) return;
+  int dlo, dhi, items[kMaxSplitKblk], longest = 0;
+  band_offsets(a->causal != 0, a->has_window != 0, clamp_window(a->window_left), clamp_window(a->window_right), dlo, dhi);
+  int64_t total = 0;
+  for (int k = 0; k < nk; ++k) {
+    items[k] = bwd_kv_items(k, BK, G, (int)a->seqlen_q, (int)a->seqlen_k, dlo, dhi, BQ);
+    longest = std::max(longest, items[k]);
+    total += items[k];
+  }
+  if (longest < 2) return;
+  const double item_us = D == 128 ? 1.7 : 1.0, piece_us = 2.0 * BK * D * 2 * 4 / 4e6;
+  const double share = (double)total * groups / slots;
+  // nearly equal blocks run in rounds; unequal ones, longest first, pack well
+  double whole = std::max((double)longest, 1.1 * share);
+  if (longest * (double)nk <= 1.15 * total) whole = (double)longest * ((groups * nk + slots - 1) / slots);
+  double best = 0.9 * whole;
+  for (int rounds = 1; rounds <= 2; ++rounds) {
+    int T = std::max(1, (int)(share / rounds));
+    for (; T < longest; T += std::max(1, T / 16)) {
+      int64_t pieces = 0, partial = 0;
+      for (int k = 0; k < nk; ++k) {
+        const int np = bwd_pieces(items[k], T);
+        pieces += np;
+        partial += np > 1 ? np : 0;
+      }
+      if (pieces * groups > slots * rounds) continue;
+      const double cost = (double)T * rounds + (7.0 + partial * groups * piece_us) / item_us;
+      if (cost < best) {
+        best = cost;
+        pl->kv_T = T;
+        pl->kv_P = (int)pieces;
+      }
+      break;
+    }
+  }
+  if (pl->kv_T) pl->ws_bytes = groups * pl->kv_P * 2 * BK * (int64_t)D * 4;
+}
+
+int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl, bool split) {
   const bool f32 = a->dtype == TRINIX_F32;
   const int64_t D = a->head_dim;
   pl->generic = f32 || D == 256;
@@ -322,6 +381,25 @@ int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl) {
   if (a->batch * a->nheads_q * pl->num_mblk * pl->dq_hs >= (1ll << 31) ||
       a->batch * a->nheads_kv * pl->num_kblk * pl->kv_hs >= (1ll << 31))
     return TRINIX_ERR_BAD_SHAPE;
+  pl->kv_T = pl->kv_P = 0;
+  pl->ws_bytes = 0;
+  if (split && !pl->generic) {
+    if (const char* env = getenv("TRINIX_BWD_PIECES")) {  // pieces of at most this many items, 0: whole (tuning and tests)
+      const int T = atoi(env);
+      if (T > 0 && pl->num_kblk <= kMaxSplitKblk) {
+        int dlo, dhi;
+        band_offsets(a->causal != 0, a->has_window != 0, clamp_window(a->window_left), clamp_window(a->window_right), dlo,
+                     dhi);
+        for (int k = 0; k < pl->num_kblk; ++k)
+          pl->kv_P += bwd_pieces(bwd_kv_items(k, 128, (int)(a->nheads_q / a->nheads_kv), (int)a->seqlen_q,
+                                              (int)a->seqlen_k, dlo, dhi, 64), T);
+        pl->kv_T = T;
+        pl->ws_bytes = a->batch * a->nheads_kv * pl->kv_P * 2 * 128 * D * 4;
+      }
+    } else {
+      plan_bwd_pieces(a, pl);
+    }
+  }
   return TRINIX_OK;
 }
 

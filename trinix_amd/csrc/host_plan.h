@@ -76,8 +76,16 @@ struct BwdPlan {
   bool dq_wide;
   bool generic;
   int dq_ks, kv_ks, dq_hs, kv_hs;
+  // dK/dV in pieces of at most kv_T items (0: whole key blocks), kv_P of them
+  // per (batch, KV head); the fp32 partials take ws_bytes of workspace
+  int kv_T, kv_P;
+  int64_t ws_bytes;
 };
-int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl);
+// Key blocks of a (batch, KV head) that a split plan covers: a wavefront
+// counts their pieces, one lane each.
+constexpr int kMaxSplitKblk = 64;
+// `split`: the caller has workspace for dK/dV in pieces.
+int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl, bool split = false);
 
 // Split-KV decode plan.
 constexpr int kDecodeMaxSq = 16;

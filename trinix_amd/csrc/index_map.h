@@ -230,6 +230,38 @@ __host__ __device__ inline void bwd_query_tiles(int kb0, int BK, int Sq, int Sk,
   qt_hi = i_hi > i_lo ? (i_hi + BQ - 1) / BQ : qt_lo;
 }
 
+// dK/dV in pieces.  A key block's items (query tiles of every q-head of the
+// group) are cut into bwd_pieces(n, T) nearly equal runs of at most T, each a
+// work item of its own; a block of more than one piece is summed from fp32
+// partials.  `group` = b * Hkv + hkv; `index` numbers the pieces of a group
+// over its key blocks in ascending order (longest blocks first when causal).
+// Groups are dealt to the XCDs as in bwd_kv_item.
+__host__ __device__ inline int bwd_pieces(int n_items, int T) { return n_items <= T ? 1 : (n_items + T - 1) / T; }
+// Items of key block kblk.
+__host__ __device__ inline int bwd_kv_items(int kblk, int BK, int G, int Sq, int Sk, int dlo, int dhi, int BQ) {
+  int lo, hi;
+  bwd_query_tiles(kblk * BK, BK, Sq, Sk, dlo, dhi, BQ, lo, hi);
+  return hi > lo ? G * (hi - lo) : 0;
+}
+struct KvPiece {
+  int group, index;
+};
+__host__ __device__ inline KvPiece bwd_kv_piece(int blk, int groups, int per_group) {
+  KvPiece pc;
+  if (groups % kXcds == 0) {
+    const int xcd = blk % kXcds, j = blk / kXcds, ng = groups / kXcds;
+    pc.index = j / ng;
+    pc.group = xcd * ng + j % ng;
+  } else {
+    const int w = xcd_remap(blk, groups * per_group);
+    pc.index = w % per_group;
+    pc.group = w / per_group;
+  }
+  return pc;
+}
+// First item of piece `k` of np (items [first(k), first(k + 1)) of n).
+__host__ __device__ inline int bwd_piece_first(int n_items, int np, int k) { return (int)((int64_t)n_items * k / np); }
+
 // dQ: work item (batch, kv-head, q-head in the group, first row m0) of
 // workgroup `blk`, rows in blocks of BM (causal: longest rows first).
 struct DqItem {

@@ -351,7 +351,7 @@ def _launch_cached(key, q, k, v, rotary_cos, rotary_sin):
 # (and keep map) per call as on the full path.
 class _TrainLaunch:
     __slots__ = ("fwd", "bwd", "out_shape", "lse_shape", "dtype", "device", "align", "km_bytes", "do_stride",
-                 "dk_shape")
+                 "dk_shape", "ws_bytes")
 
     def __init__(self, fwd, out_shape, lse_shape, dtype, device, align, km_bytes, dk_shape):
         self.fwd = fwd                # AttnFwdArgs with null data pointers and seed
@@ -364,6 +364,7 @@ class _TrainLaunch:
         self.km_bytes = km_bytes      # dropout keep map bytes (0: none)
         self.do_stride = None         # dout strides the backward template was built for
         self.dk_shape = dk_shape      # shape of k (and of dk, dv)
+        self.ws_bytes = 0             # workspace of the backward
 
 
 _TRAIN_LAUNCHES: dict = {}
@@ -652,6 +653,18 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
     return out, lse, state
 
 
+def _launch_bwd(a, ws_bytes, device):
+    """``trinix_attn_bwd``, with a workspace for dK/dV in pieces where the plan
+    asks for one (kept alive by the allocator's stream order)."""
+    lib = nat.load_library()
+    if ws_bytes:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+        nat.check(lib.trinix_attn_bwd_ws(ctypes.byref(a), ws.data_ptr(), ws_bytes, current_stream_ptr(device)),
+                  "trinix_attn_bwd_ws")
+    else:
+        nat.check(lib.trinix_attn_bwd(ctypes.byref(a), current_stream_ptr(device)), "trinix_attn_bwd")
+
+
 def _backward(state, dout):
     """Launch ``trinix_attn_bwd`` for a forward run with ``keep_state``;
     returns (dq, dk, dv) at the caller's head_dim, in the input dtype."""
@@ -690,14 +703,17 @@ def _backward(state, dout):
         a.dropout_state = state["dropout_state"].data_ptr()
     if state["keep_map"] is not None:
         a.dropout_keep_map = state["keep_map"].data_ptr()
-    rc = nat.load_library().trinix_attn_bwd(ctypes.byref(a), current_stream_ptr(qk.device))
-    nat.check(rc, "trinix_attn_bwd")
+    wsb = ctypes.c_int64(0)
+    nat.check(nat.load_library().trinix_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(wsb)),
+              "trinix_attn_bwd_workspace")
+    _launch_bwd(a, wsb.value, qk.device)
     if ent is not None and ent.bwd is None and do is dout and state["dropout_state"] is None:
         tpl = nat.AttnBwdArgs.from_buffer_copy(a)
         tpl.q = tpl.k = tpl.v = tpl.out = tpl.dout = tpl.lse = tpl.delta = tpl.dq = tpl.dk = tpl.dv = None
         tpl.dropout_keep_map = None
         tpl.dropout_seed = 0
         ent.do_stride = tuple(do.stride())
+        ent.ws_bytes = wsb.value
         ent.bwd = tpl
     if dkrn != D:
         dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
@@ -722,7 +738,7 @@ def _backward_cached(state, ent, dout):
         a.dropout_seed = state["dropout"][1]
         if state["keep_map"] is not None:
             a.dropout_keep_map = state["keep_map"].data_ptr()
-    nat.check(nat.load_library().trinix_attn_bwd(ctypes.byref(a), current_stream_ptr(dev)), "trinix_attn_bwd")
+    _launch_bwd(a, ent.ws_bytes, dev)
     return dq, dk, dv
 
 
