@@ -383,6 +383,25 @@ int trinix_attn_bwd(const trinix_attn_bwd_args* args, void* stream);
 int trinix_attn_bwd_workspace(const trinix_attn_bwd_args* args, int64_t* workspace_bytes);
 int trinix_attn_bwd_ws(const trinix_attn_bwd_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Head dims between the kernels' (the reference pads them,
+ * trinix/kernels/utils.py:107): q, k and v zero-padded to args->head_dim
+ * (trinix_pad_heads), the other tensors at their own d_out columns.  bf16 /
+ * fp16, args->head_dim 64 or 128, d_out a multiple of 8 (equal to head_dim: the
+ * plain entry points); without fused RoPE or q norm.
+ * trinix_attn_fwd_narrow writes d_out columns of out.  trinix_attn_bwd_narrow
+ * reads d_out columns of out and dout and writes d_out columns of dq, dk and dv;
+ * its workspace (trinix_attn_bwd_narrow_workspace) also holds a padded dout. */
+int trinix_attn_fwd_narrow(const trinix_attn_fwd_args* args, int64_t d_out, void* stream);
+int trinix_attn_bwd_narrow_workspace(const trinix_attn_bwd_args* args, int64_t d_out, int64_t* workspace_bytes);
+int trinix_attn_bwd_narrow(const trinix_attn_bwd_args* args, int64_t d_out, void* workspace, int64_t workspace_bytes,
+                           void* stream);
+/* Zero-pads the rows of n = 1..3 (B, S, H, head_dim) 16-bit tensors to out_dim
+ * columns (a multiple of 8) in one launch: tensor k at x[k] with element
+ * strides x_stride[4k..] (last one 1), sizes[3k..] = B, S, H, into the
+ * contiguous (B, S, H, out_dim) out[k] (16-byte aligned). */
+int trinix_pad_heads(int32_t n, const void* const* x, const int64_t* x_stride, void* const* out, const int64_t* sizes,
+                     int64_t head_dim, int64_t out_dim, int32_t dtype, void* stream);
+
 /* ALiBi bias, reference trinix/kernels/alibi_kernel.py:8-54:
  *   out[h*out_stride_h + i*out_stride_i + j] = -slopes[h*slope_stride] * |i - j|
  * for h < nheads, i, j < seqlen (< 2^24), fp32, key stride 1. */

@@ -171,6 +171,10 @@ SIGNATURES = {
     "trinix_attn_bwd": (c_int32, [POINTER(AttnBwdArgs), c_void_p]),
     "trinix_attn_bwd_workspace": (c_int32, [POINTER(AttnBwdArgs), POINTER(c_int64)]),
     "trinix_attn_bwd_ws": (c_int32, [POINTER(AttnBwdArgs), c_void_p, c_int64, c_void_p]),
+    "trinix_attn_fwd_narrow": (c_int32, [POINTER(AttnFwdArgs), c_int64, c_void_p]),
+    "trinix_attn_bwd_narrow_workspace": (c_int32, [POINTER(AttnBwdArgs), c_int64, POINTER(c_int64)]),
+    "trinix_attn_bwd_narrow": (c_int32, [POINTER(AttnBwdArgs), c_int64, c_void_p, c_int64, c_void_p]),
+    "trinix_pad_heads": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_void_p]),
     "trinix_qk_norm": (
         c_int32,
         [c_void_p, POINTER(c_int64), c_void_p, POINTER(c_int64), c_int64, c_int64, c_int64, c_int64, c_int32,

@@ -20,7 +20,7 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const uint16_t* __restri
                                                         int64_t o_sh, const uint16_t* __restrict__ dout, int64_t do_sb,
                                                         int64_t do_ss, int64_t do_sh, const float* __restrict__ lse,
                                                         float* __restrict__ delta, float dmul, int Hq, int Sq,
-                                                        int64_t rows) {
+                                                        int64_t rows, int d_out, uint16_t* __restrict__ dout_pad) {
   constexpr int LPR = D / 8, RPB = 256 / LPR;
   const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
   const int t = threadIdx.x % LPR;
@@ -30,8 +30,13 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const uint16_t* __restri
     const int64_t bh = row / Sq;
     const int h = (int)(bh % Hq);
     const int64_t b = bh / Hq;
-    const u32x4_t ov = *(const u32x4_t*)(o + b * o_sb + i * o_ss + h * o_sh + t * 8);
-    const u32x4_t dv = *(const u32x4_t*)(dout + b * do_sb + i * do_ss + h * do_sh + t * 8);
+    u32x4_t ov = {}, dv = {};
+    if (t * 8 < d_out) {
+      ov = *(const u32x4_t*)(o + b * o_sb + i * o_ss + h * o_sh + t * 8);
+      dv = *(const u32x4_t*)(dout + b * do_sb + i * do_ss + h * do_sh + t * 8);
+    }
+    // narrower out and dout: leave dout zero-padded for the gradient kernels
+    if (dout_pad) *(u32x4_t*)(dout_pad + ((b * Sq + i) * Hq + h) * D + t * 8) = dv;
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc += E::lo(ov[e]) * E::lo(dv[e]) + E::hi(ov[e]) * E::hi(dv[e]);
   }
@@ -86,7 +91,17 @@ hipError_t launch_delta(const BwdParams& p, hipStream_t st) {
   const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
   return launch_kernel(&bwd_delta_kernel<E, D>, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st, p.o,
                        p.o_sb, p.o_ss, p.o_sh, p.dout, p.do_sb, p.do_ss, p.do_sh, p.lse, p.delta,
-                       p.use_dropout ? 1.f / p.drop_scale : 1.f, p.Hq, p.Sq, rows);
+                       p.use_dropout ? 1.f / p.drop_scale : 1.f, p.Hq, p.Sq, rows, p.d_out, p.dout_pad);
+}
+
+// The gradient kernels read dout at head_dim: after the delta pass, the
+// padded copy it left.
+void use_padded_dout(BwdParams& p, int D) {
+  if (!p.dout_pad) return;
+  p.dout = p.dout_pad;
+  p.do_sh = D;
+  p.do_ss = (int64_t)p.Hq * D;
+  p.do_sb = p.do_ss * p.Sq;
 }
 
 }  // namespace
@@ -96,9 +111,17 @@ using namespace trinix;
 
 namespace {
 
-int run_bwd(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_bytes, bool split, void* stream) {
+// Bytes of the padded dout copy of a narrow call, a multiple of 16.
+int64_t pad_bytes(const trinix_attn_bwd_args* a) { return a->batch * a->seqlen_q * a->nheads_q * a->head_dim * 2; }
+
+// d_out < head_dim: the narrow entry point (its padded dout at the front of
+// the workspace).
+int run_bwd(const trinix_attn_bwd_args* a, int64_t d_out, void* workspace, int64_t workspace_bytes, bool split,
+            void* stream) {
   const int vrc = validate_bwd_args(a);
   if (vrc != TRINIX_OK) return vrc;
+  const int nrc = check_narrow(a->dtype, a->head_dim, d_out);
+  if (nrc != TRINIX_OK) return nrc;
 
   BwdParams p{};
   p.q = (const uint16_t*)a->q;
@@ -144,11 +167,15 @@ int run_bwd(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_by
   BwdPlan plan;
   const int prc = plan_bwd(a, &plan, split);
   if (prc != TRINIX_OK) return prc;
-  if (plan.ws_bytes > 0 && (!workspace || workspace_bytes < plan.ws_bytes || ((uintptr_t)workspace & 15) != 0))
+  const int64_t pad = d_out < a->head_dim ? pad_bytes(a) : 0;
+  if (plan.ws_bytes + pad > 0 &&
+      (!workspace || workspace_bytes < plan.ws_bytes + pad || ((uintptr_t)workspace & 15) != 0))
     return TRINIX_ERR_BAD_ARGUMENT;
+  p.d_out = (int)d_out;
+  p.dout_pad = pad ? (uint16_t*)workspace : nullptr;
   p.kv_T = plan.kv_T;
   p.kv_P = plan.kv_P;
-  p.part = (float*)workspace;
+  p.part = plan.ws_bytes ? (float*)((char*)workspace + pad) : nullptr;
   p.num_kblk = plan.num_kblk;
   p.num_mblk = plan.num_mblk;
   p.dq_wide = plan.dq_wide ? 1 : 0;
@@ -185,9 +212,11 @@ int run_bwd(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_by
     if (err == hipSuccess) err = bf ? launch_bwd_generic_bf16(p, plan, st) : launch_bwd_generic_f16(p, plan, st);
   } else if (a->head_dim == 128) {
     err = bf ? launch_delta<BF16, 128>(p, st) : launch_delta<F16, 128>(p, st);
+    use_padded_dout(p, 128);
     if (err == hipSuccess) err = bf ? launch_bwd16_bf16_d128(p, feat, st) : launch_bwd16_f16_d128(p, feat, st);
   } else {
     err = bf ? launch_delta<BF16, 64>(p, st) : launch_delta<F16, 64>(p, st);
+    use_padded_dout(p, 64);
     if (err == hipSuccess) err = bf ? launch_bwd16_bf16_d64(p, feat, st) : launch_bwd16_f16_d64(p, feat, st);
   }
   return err == hipSuccess ? TRINIX_OK : TRINIX_ERR_LAUNCH;
@@ -195,7 +224,9 @@ int run_bwd(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_by
 
 }  // namespace
 
-extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) { return run_bwd(a, nullptr, 0, false, stream); }
+extern "C" int trinix_attn_bwd(const trinix_attn_bwd_args* a, void* stream) {
+  return run_bwd(a, a ? a->head_dim : 0, nullptr, 0, false, stream);
+}
 
 extern "C" int trinix_attn_bwd_workspace(const trinix_attn_bwd_args* a, int64_t* bytes) {
   if (!bytes) return TRINIX_ERR_NULL_POINTER;
@@ -209,5 +240,18 @@ extern "C" int trinix_attn_bwd_workspace(const trinix_attn_bwd_args* a, int64_t*
 }
 
 extern "C" int trinix_attn_bwd_ws(const trinix_attn_bwd_args* a, void* workspace, int64_t workspace_bytes, void* stream) {
-  return run_bwd(a, workspace, workspace_bytes, true, stream);
+  return run_bwd(a, a ? a->head_dim : 0, workspace, workspace_bytes, true, stream);
+}
+
+extern "C" int trinix_attn_bwd_narrow_workspace(const trinix_attn_bwd_args* a, int64_t d_out, int64_t* bytes) {
+  const int rc = trinix_attn_bwd_workspace(a, bytes);
+  if (rc != TRINIX_OK) return rc;
+  const int nrc = check_narrow(a->dtype, a->head_dim, d_out);
+  if (nrc == TRINIX_OK && d_out < a->head_dim) *bytes += pad_bytes(a);
+  return nrc;
+}
+
+extern "C" int trinix_attn_bwd_narrow(const trinix_attn_bwd_args* a, int64_t d_out, void* workspace,
+                                      int64_t workspace_bytes, void* stream) {
+  return run_bwd(a, d_out, workspace, workspace_bytes, true, stream);
 }

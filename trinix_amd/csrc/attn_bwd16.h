@@ -72,6 +72,10 @@ struct BwdParams {
   // (batch, KV head); fp32 partials of the key blocks of several pieces
   int kv_T, kv_P;
   float* part;
+  // columns of out and dout read and of dq, dk, dv written (head_dim, or
+  // fewer: q, k, v zero-padded to head_dim); then dout_pad takes dout padded
+  int d_out;
+  uint16_t* dout_pad;
   int rows16;                  // fp32: q, k, v and dout take 16-byte copies (rows_aligned16)
 };
 
@@ -280,7 +284,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce(const BwdParams p) {
   f32x4_t s = *(const f32x4_t*)part;
   for (int k = 1; k < hi - lo; ++k) s += *(const f32x4_t*)(part + (int64_t)k * 2 * BK * D);
   const int j = kblk * BK + kg * 32 + (l & 31), d0 = dq * 8 + (l >> 5) * 4;
-  if (j >= p.Sk) return;
+  if (j >= p.Sk || d0 >= p.d_out) return;
   const int b = group / p.Hkv, hkv = group % p.Hkv;
   uint16_t* row = sb ? p.dk + b * p.dk_sb + hkv * p.dk_sh + (int64_t)j * p.dk_ss
                      : p.dv + b * p.dv_sb + hkv * p.dv_sh + (int64_t)j * p.dv_ss;
@@ -705,6 +709,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq) {
           const int d0 = db * 32 + vq * 8 + g * 4;
+          if (d0 >= p.d_out) continue;  // columns of zero padding
           *(u32x2_t*)(row + d0) = (u32x2_t){E::pack(acc[db][vq * 4 + 0] * f, acc[db][vq * 4 + 1] * f),
                                             E::pack(acc[db][vq * 4 + 2] * f, acc[db][vq * 4 + 3] * f)};
         }
@@ -1012,6 +1017,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_bwd_dq(const BwdParams p) {
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
         const int d0 = db * 32 + vq * 8 + g * 4;
+        if (d0 >= p.d_out) continue;  // columns of zero padding
         *(u32x2_t*)(qrow + d0) = (u32x2_t){E::pack(acc[db][vq * 4 + 0] * f, acc[db][vq * 4 + 1] * f),
                                            E::pack(acc[db][vq * 4 + 2] * f, acc[db][vq * 4 + 3] * f)};
       }

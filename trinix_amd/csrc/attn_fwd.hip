@@ -87,8 +87,15 @@ int trinix_attn_tile_config(int64_t head_dim, int32_t dtype, trinix_tile_cfg* ou
 }
 
 int trinix_attn_fwd(const trinix_attn_fwd_args* a, void* stream) {
+  return trinix_attn_fwd_narrow(a, a ? a->head_dim : 0, stream);
+}
+
+int trinix_attn_fwd_narrow(const trinix_attn_fwd_args* a, int64_t d_out, void* stream) {
   const int vrc = validate_fwd_args(a);
   if (vrc != TRINIX_OK) return vrc;
+  const int nrc = check_narrow(a->dtype, a->head_dim, d_out);
+  if (nrc != TRINIX_OK) return nrc;
+  if (d_out < a->head_dim && (a->q_norm_weight || a->rope_cos)) return TRINIX_ERR_BAD_ARGUMENT;  // over head_dim columns
 
   FwdParams p{};  // value-initialised: fields a configuration does not use are zero
   p.q = (const uint16_t*)a->q;
@@ -148,6 +155,7 @@ int trinix_attn_fwd(const trinix_attn_fwd_args* a, void* stream) {
   p.qn_eps = a->q_norm_eps;
   p.qn_out = (uint16_t*)a->q_norm_out;
   p.keep_map = (uint32_t*)a->dropout_keep_map;
+  p.d_out = (int)d_out;
   p.km_nbi = keep_map_nbi(a->seqlen_q);
   p.km_nbj = keep_map_nbj(a->seqlen_k);
 

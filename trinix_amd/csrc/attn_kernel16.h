@@ -723,6 +723,7 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
         const int d0 = db * 32 + vq * 8 + ge * 4;
+        if (d0 >= p.d_out) continue;  // columns of zero padding
         const u32x2_t w2 = {E::pack(acc[db][vq * 4 + 0] * inv, acc[db][vq * 4 + 1] * inv),
                             E::pack(acc[db][vq * 4 + 2] * inv, acc[db][vq * 4 + 3] * inv)};
         *(u32x2_t*)(orow + d0) = w2;

@@ -45,6 +45,7 @@ struct FwdParams {
   uint16_t* qn_out;  // the normalised q, contiguous (B, Sq, Hq, D), or null
   uint32_t* keep_map;    // dropout keep bits written for the backward (index_map.h), or null
   int64_t km_nbi, km_nbj;  // its row / key blocks per (batch, q-head)
+  int d_out;               // columns of out written (16-bit; head_dim, or fewer: zero-padded q, k, v)
   int rows16;              // fp32: k and v take 16-byte copies (rows_aligned16)
   // work items of the per-item key split (Cfg16 ks = 0), longest chain
   // first: row block << 2 | split << 1 | half (plan_split_rows)

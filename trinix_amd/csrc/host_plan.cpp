@@ -242,6 +242,13 @@ int validate_bwd_args(const trinix_attn_bwd_args* a) {
   return TRINIX_OK;
 }
 
+int check_narrow(int32_t dtype, int64_t head_dim, int64_t d_out) {
+  if (d_out == head_dim) return TRINIX_OK;
+  const bool ok = (dtype == TRINIX_BF16 || dtype == TRINIX_F16) && (head_dim == 64 || head_dim == 128) && d_out > 0 &&
+                  d_out < head_dim && d_out % 8 == 0;
+  return ok ? TRINIX_OK : TRINIX_ERR_BAD_HEAD_DIM;
+}
+
 int64_t clamp_window(int64_t w) {
   const int64_t lim = 1ll << 30;
   return w < -lim ? -lim : (w > lim ? lim : w);

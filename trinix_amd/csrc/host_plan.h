@@ -28,6 +28,9 @@ constexpr int64_t kMaxKvRowStride = 1ll << 22;
 // trinix_attn_bwd: TRINIX_OK or the status code to return, no launch.
 int validate_fwd_args(const trinix_attn_fwd_args* a);
 int validate_bwd_args(const trinix_attn_bwd_args* a);
+// d_out of the narrow entry points: head_dim, or for the 16-bit kernels at
+// head_dim 64 and 128 a smaller multiple of 8.
+int check_narrow(int32_t dtype, int64_t head_dim, int64_t d_out);
 
 // Tile configuration of the 16-bit forward for a problem: `banded` when
 // causal or windowed, `plain` without a mask or dropout, `split_ok` when the

@@ -99,6 +99,28 @@ def _prepare_operand(t: torch.Tensor, d_kernel: int) -> torch.Tensor:
     return t
 
 
+class _Pad:
+    """One ``trinix_pad_heads`` launch of q, k and v of a layout: their strides
+    and sizes, apart from the data pointers."""
+
+    __slots__ = ("strides", "sizes", "shapes", "head_dim", "d_kernel", "dtype", "code")
+
+    def __init__(self, ts, d_kernel):
+        self.strides = (ctypes.c_int64 * 12)(*(st for t in ts for st in t.stride()))
+        self.sizes = (ctypes.c_int64 * 9)(*(n for t in ts for n in t.shape[:3]))
+        self.shapes = [(*t.shape[:3], d_kernel) for t in ts]
+        self.head_dim, self.d_kernel = ts[0].shape[-1], d_kernel
+        self.dtype, self.code = ts[0].dtype, _DTYPE_CODE[ts[0].dtype]
+
+    def __call__(self, ts, device, stream):
+        outs = [torch.empty(sh, dtype=self.dtype, device=device) for sh in self.shapes]
+        nat.check(nat.load_library().trinix_pad_heads(
+            3, (ctypes.c_void_p * 3)(*(t.data_ptr() for t in ts)), self.strides,
+            (ctypes.c_void_p * 3)(*(o.data_ptr() for o in outs)), self.sizes, self.head_dim, self.d_kernel, self.code,
+            stream), "trinix_pad_heads")
+        return outs
+
+
 class TritonAttentionKernel:
     """MI355X attention forward (name kept from the reference for drop-in use).
 
@@ -275,9 +297,9 @@ def _keep_map_bytes(device: torch.device, B: int, H: int, Sq: int, Sk: int) -> i
 # leaves a template, so the errors of the full path are unchanged.
 # ---------------------------------------------------------------------------
 class _Launch:
-    __slots__ = ("args", "out_shape", "dtype", "device", "align", "rope", "split")
+    __slots__ = ("args", "out_shape", "dtype", "device", "align", "rope", "split", "pad")
 
-    def __init__(self, args, out_shape, dtype, device, align, rope, split):
+    def __init__(self, args, out_shape, dtype, device, align, rope, split, pad=None):
         self.args = args            # AttnFwdArgs with null data pointers
         self.out_shape = out_shape
         self.dtype = dtype
@@ -285,6 +307,7 @@ class _Launch:
         self.align = align          # byte alignment the operand pointers need
         self.rope = rope            # k pre-pass: (k_stride, out_stride, B, S, H, D, cs_stride, rows) or None
         self.split = split          # split-KV workspace bytes, or None for trinix_attn_fwd
+        self.pad = pad              # _Pad of q, k and v (a head_dim between the kernels'), or None
 
 
 _LAUNCHES: dict = {}
@@ -325,6 +348,12 @@ def _launch_cached(key, q, k, v, rotary_cos, rotary_sin):
     lib = nat.load_library()
     stream = current_stream_ptr(ent.device)
     a = nat.AttnFwdArgs.from_buffer_copy(ent.args)
+    if ent.pad is not None:
+        out = torch.empty(ent.out_shape, dtype=ent.dtype, device=ent.device)
+        padded = ent.pad((q, k, v), ent.device, stream)
+        a.q, a.k, a.v, a.out = *(t.data_ptr() for t in padded), out.data_ptr()
+        nat.check(lib.trinix_attn_fwd_narrow(ctypes.byref(a), ent.pad.head_dim, stream), "trinix_attn_fwd_narrow")
+        return out
     if ent.rope is not None:
         ks, os_, B, S, H, D, cs_stride, rows = ent.rope
         kr = torch.empty((B, S, H, D), dtype=ent.dtype, device=ent.device)
@@ -345,15 +374,16 @@ def _launch_cached(key, q, k, v, rotary_cos, rotary_sin):
 
 # Training launches.  A differentiable call (the forward keeps state for the
 # backward) without mask, ALiBi, q-norm or fused rotary tables, whose
-# operands the kernels read in place, is cached the same way: the forward's
+# operands the kernels (or the padding launch of a head_dim between theirs)
+# read in place, is cached the same way: the forward's
 # argument template (its lse written) and, once the first backward of the
 # layout has run, the backward's template.  Dropout calls draw their seed
 # (and keep map) per call as on the full path.
 class _TrainLaunch:
     __slots__ = ("fwd", "bwd", "out_shape", "lse_shape", "dtype", "device", "align", "km_bytes", "do_stride",
-                 "dk_shape", "ws_bytes")
+                 "dk_shape", "ws_bytes", "pad", "do_align")
 
-    def __init__(self, fwd, out_shape, lse_shape, dtype, device, align, km_bytes, dk_shape):
+    def __init__(self, fwd, out_shape, lse_shape, dtype, device, align, km_bytes, dk_shape, pad, do_align):
         self.fwd = fwd                # AttnFwdArgs with null data pointers and seed
         self.bwd = None               # AttnBwdArgs template after the first backward, or None
         self.out_shape = out_shape
@@ -365,6 +395,8 @@ class _TrainLaunch:
         self.do_stride = None         # dout strides the backward template was built for
         self.dk_shape = dk_shape      # shape of k (and of dk, dv)
         self.ws_bytes = 0             # workspace of the backward
+        self.pad = pad                # _Pad of q, k and v (a head_dim between the kernels'), or None
+        self.do_align = do_align      # byte alignment dout needs
 
 
 _TRAIN_LAUNCHES: dict = {}
@@ -397,11 +429,16 @@ def _train_cached(tkey, q, k, v):
             a.dropout_keep_map = keep_map.data_ptr()
     out = torch.empty(ent.out_shape, dtype=ent.dtype, device=ent.device)
     lse = torch.empty(ent.lse_shape, dtype=torch.float32, device=ent.device)
-    a.q, a.k, a.v, a.out, a.lse = qp, kp, vp, out.data_ptr(), lse.data_ptr()
-    nat.check(nat.load_library().trinix_attn_fwd(ctypes.byref(a), current_stream_ptr(ent.device)), "trinix_attn_fwd")
-    D = ent.out_shape[-1]
-    state = dict(q=q, k=k, v=v, out=out, lse=lse, D=D, d_kernel=D, args=a, launch=ent,
-                 dropout=(float(a.dropout_p), int(a.dropout_seed), 0), dropout_state=None, keep_map=keep_map)
+    lib, stream, D = nat.load_library(), current_stream_ptr(ent.device), ent.out_shape[-1]
+    if ent.pad is None:
+        a.q, a.k, a.v, a.out, a.lse = qp, kp, vp, out.data_ptr(), lse.data_ptr()
+        nat.check(lib.trinix_attn_fwd(ctypes.byref(a), stream), "trinix_attn_fwd")
+    else:
+        q, k, v = ent.pad((q, k, v), ent.device, stream)
+        a.q, a.k, a.v, a.out, a.lse = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr()
+        nat.check(lib.trinix_attn_fwd_narrow(ctypes.byref(a), D, stream), "trinix_attn_fwd_narrow")
+    state = dict(q=q, k=k, v=v, out=out, lse=lse, D=D, d_kernel=int(a.head_dim), narrow=ent.pad is not None, args=a,
+                 launch=ent, dropout=(float(a.dropout_p), int(a.dropout_seed), 0), dropout_state=None, keep_map=keep_map)
     return out, lse, state
 
 
@@ -490,10 +527,19 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
         q = rope_apply(q, rotary_cos, rotary_sin)
         rotary_cos = rotary_sin = None
 
-    qk = _prepare_operand(q, d_kernel)
-    kk = _prepare_operand(k, d_kernel)
-    vk = _prepare_operand(v, d_kernel)
-    out = torch.empty((B, Sq, H, d_kernel), dtype=q.dtype, device=device)
+    pad = None
+    if d_kernel != D and q.dtype != torch.float32:
+        # zero-padded in one launch; where the kernels can, they read and
+        # write the other tensors at their own D columns ("narrow")
+        ts = tuple(t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
+        pad = _Pad(ts, d_kernel)
+        qk, kk, vk = pad(ts, device, stream)
+    else:
+        qk = _prepare_operand(q, d_kernel)
+        kk = _prepare_operand(k, d_kernel)
+        vk = _prepare_operand(v, d_kernel)
+    narrow = pad is not None and d_kernel <= 128 and D % 8 == 0 and not split_kv
+    out = torch.empty((B, Sq, H, D if narrow else d_kernel), dtype=q.dtype, device=device)
 
     args = nat.AttnFwdArgs()
     args.q, args.k, args.v, args.out = qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr()
@@ -614,9 +660,19 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
             nat.check(rc, "trinix_attn_fwd_splitkv")
             launched = True
             split_bytes = wsb.value
-    if not launched:
+    if not launched and narrow:
+        nat.check(lib.trinix_attn_fwd_narrow(ctypes.byref(args), D, stream), "trinix_attn_fwd_narrow")
+    elif not launched:
         rc = lib.trinix_attn_fwd(ctypes.byref(args), stream)
         nat.check(rc, "trinix_attn_fwd")
+    # q, k and v as given went through the padding launch alone
+    narrow_in_place = narrow and all(a is b for a, b in zip(ts, (q_in, k_in, v_in)))
+    if key is not None and narrow_in_place:
+        tpl = nat.AttnFwdArgs.from_buffer_copy(args)
+        tpl.q = tpl.k = tpl.v = tpl.out = None
+        if len(_LAUNCHES) >= _MAX_LAUNCHES:
+            _LAUNCHES.clear()
+        _LAUNCHES[key] = _Launch(tpl, tuple(out.shape), q.dtype, device, 2, None, None, pad)
     if key is not None and d_kernel == D:
         # the operands went to the kernel as given (no copy, no padding, q
         # not rotated ahead, tables used in place): remember the launch
@@ -635,29 +691,37 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
     state = None
     if keep_state:
         ent = None
-        if (tkey is not None and d_kernel == D and qk is q_in and kk is k_in and vk is v_in and drop_state is None
-                and q.dtype != torch.float32 and not launched):
+        in_place = d_kernel == D and qk is q_in and kk is k_in and vk is v_in
+        if tkey is not None and (in_place or narrow_in_place) and drop_state is None and not launched:
             tpl = nat.AttnFwdArgs.from_buffer_copy(args)
             tpl.q = tpl.k = tpl.v = tpl.out = tpl.lse = tpl.dropout_keep_map = None
             tpl.dropout_seed = 0
             if len(_TRAIN_LAUNCHES) >= _MAX_LAUNCHES:
                 _TRAIN_LAUNCHES.clear()
-            ent = _TrainLaunch(tpl, tuple(out.shape), tuple(lse.shape), q.dtype, device, 16,
-                               keep_map.numel() if keep_map is not None else 0, tuple(kk.shape))
+            esz = q.element_size()
+            ent = _TrainLaunch(tpl, tuple(out.shape), tuple(lse.shape), q.dtype, device,
+                               16 if esz == 2 and not narrow else esz, keep_map.numel() if keep_map is not None else 0,
+                               (*kk.shape[:3], out.shape[-1]), pad if narrow else None, 16 if esz == 2 else 4)
             _TRAIN_LAUNCHES[tkey] = ent
-        state = dict(q=qk, k=kk, v=vk, out=out, lse=lse, D=D, d_kernel=d_kernel, keep=keep, args=args, launch=ent,
+        state = dict(q=qk, k=kk, v=vk, out=out, lse=lse, D=D, d_kernel=d_kernel, narrow=narrow, keep=keep, args=args,
+                     launch=ent,
                      dropout=(float(args.dropout_p), int(args.dropout_seed), int(args.dropout_offset)),
                      dropout_state=drop_state, keep_map=keep_map)
-    if d_kernel != D:
+    if d_kernel != D and not narrow:
         out = out[..., :D].contiguous()
     return out, lse, state
 
 
-def _launch_bwd(a, ws_bytes, device):
+def _launch_bwd(a, ws_bytes, device, d_out=None):
     """``trinix_attn_bwd``, with a workspace for dK/dV in pieces where the plan
-    asks for one (kept alive by the allocator's stream order)."""
+    asks for one (kept alive by the allocator's stream order); with ``d_out``
+    the narrow entry point."""
     lib = nat.load_library()
-    if ws_bytes:
+    if d_out is not None:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+        nat.check(lib.trinix_attn_bwd_narrow(ctypes.byref(a), d_out, ws.data_ptr(), ws_bytes,
+                                             current_stream_ptr(device)), "trinix_attn_bwd_narrow")
+    elif ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
         nat.check(lib.trinix_attn_bwd_ws(ctypes.byref(a), ws.data_ptr(), ws_bytes, current_stream_ptr(device)),
                   "trinix_attn_bwd_ws")
@@ -678,10 +742,11 @@ def _backward(state, dout):
     D, dkrn = state["D"], state["d_kernel"]
     B, Sq, H, _ = qk.shape
     Sk, Hkv = kk.shape[1], kk.shape[2]
-    do = _prepare_operand(dout.to(qk.dtype), dkrn)
-    dq = torch.empty((B, Sq, H, dkrn), dtype=qk.dtype, device=qk.device)
-    dk = torch.empty((B, Sk, Hkv, dkrn), dtype=qk.dtype, device=qk.device)
-    dv = torch.empty((B, Sk, Hkv, dkrn), dtype=qk.dtype, device=qk.device)
+    d_out = D if state["narrow"] else dkrn
+    do = _prepare_operand(dout.to(qk.dtype), d_out)
+    dq = torch.empty((B, Sq, H, d_out), dtype=qk.dtype, device=qk.device)
+    dk = torch.empty((B, Sk, Hkv, d_out), dtype=qk.dtype, device=qk.device)
+    dv = torch.empty((B, Sk, Hkv, d_out), dtype=qk.dtype, device=qk.device)
     delta = torch.empty((B, H, Sq), dtype=torch.float32, device=qk.device)
     a = nat.AttnBwdArgs()
     a.q, a.k, a.v, a.out, a.dout = qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(), do.data_ptr()
@@ -704,9 +769,13 @@ def _backward(state, dout):
     if state["keep_map"] is not None:
         a.dropout_keep_map = state["keep_map"].data_ptr()
     wsb = ctypes.c_int64(0)
-    nat.check(nat.load_library().trinix_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(wsb)),
-              "trinix_attn_bwd_workspace")
-    _launch_bwd(a, wsb.value, qk.device)
+    if state["narrow"]:
+        nat.check(nat.load_library().trinix_attn_bwd_narrow_workspace(ctypes.byref(a), D, ctypes.byref(wsb)),
+                  "trinix_attn_bwd_narrow_workspace")
+    else:
+        nat.check(nat.load_library().trinix_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(wsb)),
+                  "trinix_attn_bwd_workspace")
+    _launch_bwd(a, wsb.value, qk.device, D if state["narrow"] else None)
     if ent is not None and ent.bwd is None and do is dout and state["dropout_state"] is None:
         tpl = nat.AttnBwdArgs.from_buffer_copy(a)
         tpl.q = tpl.k = tpl.v = tpl.out = tpl.dout = tpl.lse = tpl.delta = tpl.dq = tpl.dk = tpl.dv = None
@@ -715,7 +784,7 @@ def _backward(state, dout):
         ent.do_stride = tuple(do.stride())
         ent.ws_bytes = wsb.value
         ent.bwd = tpl
-    if dkrn != D:
+    if d_out != D:
         dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
     return dq, dk, dv
 
@@ -723,7 +792,7 @@ def _backward(state, dout):
 def _backward_cached(state, ent, dout):
     """(dq, dk, dv) through the layout's backward template, or None when
     dout is not laid out as the template's."""
-    if dout.dtype != ent.dtype or dout.stride() != ent.do_stride or dout.data_ptr() % ent.align:
+    if dout.dtype != ent.dtype or dout.stride() != ent.do_stride or dout.data_ptr() % ent.do_align:
         return None
     dev = ent.device
     a = nat.AttnBwdArgs.from_buffer_copy(ent.bwd)
@@ -738,7 +807,7 @@ def _backward_cached(state, ent, dout):
         a.dropout_seed = state["dropout"][1]
         if state["keep_map"] is not None:
             a.dropout_keep_map = state["keep_map"].data_ptr()
-    _launch_bwd(a, ent.ws_bytes, dev)
+    _launch_bwd(a, ent.ws_bytes, dev, None if ent.pad is None else ent.pad.head_dim)
     return dq, dk, dv
 
 
