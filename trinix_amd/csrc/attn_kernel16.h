@@ -65,7 +65,7 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
   constexpr int TILE_UNITS = BN * UPR;
   constexpr int LPW = TILE_UNITS / (64 * NW);  // direct loads per wavefront per tile (K or V)
   constexpr float TAU = 8.f;
-  static_assert(D % 64 == 0 && BN % 64 == 0 && TILE_UNITS % (64 * NW) == 0, "tile shape");
+  static_assert(D % 64 == 0 && BN % (MASK ? 64 : 32) == 0 && TILE_UNITS % (64 * NW) == 0, "tile shape");
 
   // Four separate LDS objects (not one array indexed by parity) so that the
   // compiler can tell the buffer being read from the one an asynchronous
@@ -207,9 +207,8 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
         }
         qr[ds] = x;
       }
-      // the q attended with, for a backward (one writer per row: the
-      // fused norm runs without the key split)
-      if (p.qn_out && i < p.Sq) {
+      // the q attended with, for a backward (one writer per row)
+      if (p.qn_out && i < p.Sq && kp == 0) {
         uint16_t* qo = p.qn_out + (((int64_t)b * p.Sq + i) * p.Hq + hq) * D;
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) *(u32x4_t*)(qo + ds * 16 + g * 8) = qr[ds];
@@ -677,15 +676,21 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
     // (m, l, O) to wavefront 2r through LDS (the K buffers are free once every
     // wavefront has passed the barrier).  Lane-for-lane: both hold the same
     // rows and head_dim columns.
-    float* mo = (float*)lds_k0;  // [row group][DB*16][64 lanes]
-    float* ml = (float*)lds_v0;  // [row group][2][64 lanes]
+    // [row group][DB*16][64 lanes]; 32-key tiles: half of the blocks in
+    // either K buffer
+    constexpr int HB = BN == 32 ? DB / 2 : DB;
+    static_assert(KS == 1 || NW / 2 * HB * 16 * 64 * 4 <= KSL * BN * D * 2, "exchange fits the K buffers");
     const int rg = wave / 2;
+    auto mo = [&](int db, int v) __attribute__((always_inline)) -> float* {
+      return (float*)(db < HB ? lds_k0 : lds_k1) + ((rg * HB + db % HB) * 16 + v) * 64 + lane;
+    };
+    float* ml = (float*)lds_v0;  // [row group][2][64 lanes]
     __syncthreads();
     if (kp == 1) {
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) mo[((rg * DB + db) * 16 + v) * 64 + lane] = acc[db][v];
+        for (int v = 0; v < 16; ++v) *mo(db, v) = acc[db][v];
       ml[(rg * 2 + 0) * 64 + lane] = m_run;
       ml[(rg * 2 + 1) * 64 + lane] = l_run;
     }
@@ -701,7 +706,7 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[db][v] = acc[db][v] * a0 + mo[((rg * DB + db) * 16 + v) * 64 + lane] * a1;
+        for (int v = 0; v < 16; ++v) acc[db][v] = acc[db][v] * a0 + *mo(db, v) * a1;
     }
   }
 
@@ -820,15 +825,20 @@ hipError_t launch_feat_split(const FwdParams& p, int feat, hipStream_t st) {
 // whose Q fragment (64 VGPRs) and O accumulator (128) need one wavefront per
 // SIMD, and whose double-buffered K/V tiles take 128 KiB of LDS; and for D = 64
 // also (4, 2, 64, 2), the key split for small grids (64 KiB of LDS: two
-// tiles per buffer), and (4, 2, 64, 0), the key split per work item.  For D = 128 without a mask or dropout also (8, 2, 128,
-// 1): 256 rows and 128-key tiles per workgroup (128 KiB of LDS, one
-// workgroup per CU).
+// tiles per buffer), and (4, 2, 64, 0), the key split per work item.  Without
+// a mask or dropout also, for D = 128, (8, 2, 128, 1): 256 rows and 128-key
+// tiles per workgroup (128 KiB of LDS, one workgroup per CU), and for D = 128
+// and 256 the key split (4, occ, 32, 2) on 32-key tiles: the LDS of the
+// unsplit shape, half its score registers per step (190 VGPRs at D = 128).
 #define TRINIX_ATTN16_LAUNCHER(NAME, E, D)                                                                   \
   hipError_t NAME(const FwdParams& p, Cfg16 cfg, int feat, hipStream_t st) {                                \
     constexpr int kOcc = (D) == 256 ? 1 : 2;                                                               \
     if constexpr ((D) == 128)                                                                              \
       if (cfg.nw == 8 && cfg.bn == 128 && cfg.occ == 2 && cfg.ks == 1)                                     \
         return launch_feat_plain<E, D, 128, 8, 2, 1>(p, feat, st);                                         \
+    if constexpr ((D) >= 128)                                                                              \
+      if (cfg.nw == 4 && cfg.bn == 32 && cfg.occ == kOcc && cfg.ks == 2)                                   \
+        return launch_feat_plain<E, D, 32, 4, kOcc, 2>(p, feat, st);                                       \
     if (cfg.bn != 64 || cfg.nw != 4 || cfg.occ != kOcc) return hipErrorNotSupported;                       \
     if (cfg.ks == 1) return launch_feat<E, D, 64, 4, kOcc, 1>(p, feat, st);                                \
     if constexpr ((D) == 64) {                                                                             \

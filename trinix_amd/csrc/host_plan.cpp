@@ -76,8 +76,28 @@ static bool wide_grid(int64_t batch, int64_t hq, int64_t sq, bool banded) {
   const int64_t need = banded ? 2 * kSmallGrid : kSmallGrid;
   return batch * hq >= need || batch * hq * ((sq + 255) / 256) >= need;
 }
+// The key split of head_dim 128 and 256 (plain features): 64-row workgroups
+// whose wavefront pairs take alternate 32-key tiles, where 128-row workgroups
+// leave CUs idle or one wavefront per SIMD, and the longest row block's
+// `chain` of 64-key tiles is worth halving against the merge.  Head_dim 128
+// runs two workgroups per CU (64 KiB of LDS), so up to one 128-row workgroup
+// per CU; head_dim 256 runs one, so up to half of that.  Measured, bf16,
+// graph-timed kernel, us without | with the split:
+//   D=128 causal, workgroups x chain: 32 x 4 9.3 | 8.8, 96 x 11 16.7 | 15.3, 120 x 6
+//     12.5 | 11.9, 240 x 10 17.2 | 16.2, 256 x 16 23.8 | 21.7, 256 x 32 39.9 |
+//     35.3, 192 x 32 40.4 | 41.0; full rows 96 x 24 31.2 | 25.8, 240 x 24 35.6 |
+//     34.1; ALiBi 256 x 32 47.2 | 41.9; where it loses: 32 x 2 7.7 | 8.0, 128 x 3
+//     8.4 | 8.8, 256 x 8 16.6 | 17.2, 384 x 16 27.9 | 30.2, 512 x 32 49.9 | 52.0
+//   D=256 48 x 11 30.0 | 25.8, 128 x 32 76.7 | 61.1, 128 x 7 windowed 27.7 | 22.9,
+//     full rows 128 x 16 49.2 | 41.5; loses: 128 x 3 14.2 | 15.2, 192 x 8 29.4 |
+//     33.1, 192 x 24 full 69.4 | 97.9
+static bool key_split(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, int64_t chain) {
+  if (head_dim < 128 || chain < 4 || batch * hq > kSmallGrid) return false;
+  const int64_t wgs = batch * hq * ((sq + 127) / 128);
+  return wgs <= kSmallGrid / 2 || (head_dim == 128 && wgs <= kSmallGrid && chain >= 10);
+}
 Cfg16 pick_cfg16(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, bool banded, bool plain,
-                 bool split_ok) {
+                 bool split_ok, int64_t chain) {
   Cfg16 c{4, head_dim == 256 ? 1 : 2, 64, 1};
   // batch * hq * row blocks, without overflow (each factor < 2^31 here)
   if (head_dim == 64 && batch * hq <= kSmallGrid && batch * hq * ((sq + 127) / 128) <= kSmallGrid) c.ks = 2;
@@ -85,6 +105,7 @@ Cfg16 pick_cfg16(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, bool b
            batch * hq * ((sq + 127) / 128) <= 2 * kSmallGrid)
     c.ks = 0;
   if (head_dim == 128 && plain && wide_grid(batch, hq, sq, banded)) c = Cfg16{8, 2, 128, 1};
+  if (plain && key_split(head_dim, batch, hq, sq, chain)) c = Cfg16{4, c.occ, 32, 2};
   if (const char* env = getenv("TRINIX_ATTN_CFG")) {
     int nw = 0, occ = 0, bn = 0, ks = 1;
     // ks 1 or 2: wavefronts per 32-row group; 0: the per-item split
@@ -274,9 +295,15 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   const bool f32 = a->dtype == TRINIX_F32;
   const bool plain = !a->mask && !(a->dropout_p > 0.f);
   const bool split_ok = plain && a->causal && !a->has_window && !a->q_norm_weight;
+  // keys the longest 128-row block sees, in 64-key tiles
+  int64_t keys = a->causal ? std::min(a->seqlen_q, a->seqlen_k) : a->seqlen_k;
+  if (a->has_window) {
+    const int64_t right = a->causal ? 0 : std::max<int64_t>(0, clamp_window(a->window_right));
+    keys = std::min(keys, std::max<int64_t>(0, clamp_window(a->window_left)) + right + 128);
+  }
   Cfg16 cfg = pick_cfg16(a->head_dim, a->batch, a->nheads_q, a->seqlen_q, a->causal || a->has_window, plain,
-                         split_ok);
-  if (a->q_norm_weight) cfg.ks = 1;  // the fused q RMSNorm is built without the key split
+                         split_ok, (keys + 63) / 64);
+  if (a->q_norm_weight && a->head_dim == 64) cfg.ks = 1;  // where the fused q RMSNorm is built without the key split
   pl->n_items = 0;
   pl->num_mblk = 0;
   pl->f32_ks = 1;
