@@ -183,13 +183,13 @@ int trinix_attn_fwd(const trinix_attn_fwd_args* args, void* stream);
  * the reference asserts seqlen_q == seqlen_k (attention_kernel.py:510) and
  * its layers' cache path runs the eager attention (base.py:347-400).
  * The rows of one KV head's q-heads are packed into 16-row tiles, and the
- * keys any row may see are cut into `num_splits` chunks merged by their
- * log-sum-exp.
+ * keys any row may see are cut into at most `num_splits` chunks merged by
+ * their log-sum-exp.
  *
  * trinix_attn_fwd_splitkv_plan: *num_splits = 0 if the split-KV kernel does
  * not apply (fp32, dropout, fused RoPE or q norm, seqlen_q > 16, no visible
  * key): use
- * trinix_attn_fwd.  Otherwise the chunk count and the size of the fp32
+ * trinix_attn_fwd.  Otherwise the largest chunk count and the size of the fp32
  * workspace trinix_attn_fwd_splitkv needs (0 for a single chunk).  Host
  * only, no launch.
  * trinix_attn_fwd_splitkv: the forward on `stream`; `workspace` is

@@ -267,6 +267,12 @@ int main() {
       check_plan(a, pl);
       CHECK(a.seqlen_q <= kDecodeMaxSq, "plan only for decode shapes");
       CHECK(pl.ws_bytes <= (int64_t)TRINIX_SPLITKV_SCRATCH_BYTES, "default plan fits the static scratch");
+      SplitPlan run = pl;
+      bool streamed;
+      decode_run_plan(&a, &run, &streamed);
+      CHECK(run.n_splits >= 1 && run.n_splits <= pl.n_splits && run.ws_bytes == pl.ws_bytes, "run within the plan");
+      run.ws_bytes = run.n_splits > 1 ? pl.ws_bytes / pl.n_splits * run.n_splits : 0;
+      check_plan(a, run);
     }
   }
   for (int it = 0; it < 50000; ++it) {
@@ -302,7 +308,14 @@ int main() {
     FwdPlan fp;
     if (plan_fwd(&f, &fp) == TRINIX_OK) bounds::model_fwd16(BR, f, fp, limit);
     SplitPlan sp;
-    if (make_split_plan(&f, &sp)) bounds::model_decode(BR, f, sp, limit);
+    if (make_split_plan(&f, &sp)) {
+      bounds::model_decode(BR, f, sp, limit);
+      const int64_t slot = sp.ws_bytes / sp.n_splits;
+      bool streamed;
+      decode_run_plan(&f, &sp, &streamed);
+      sp.ws_bytes = sp.n_splits > 1 ? slot * sp.n_splits : 0;
+      bounds::model_decode(BR, f, sp, limit);
+    }
     if (f.head_dim <= 128 && f.q_norm_weight == nullptr) {
       trinix_attn_bwd_args b = valid_bwd();
       b.batch = f.batch, b.seqlen_q = f.seqlen_q, b.seqlen_k = f.seqlen_k, b.nheads_q = f.nheads_q;

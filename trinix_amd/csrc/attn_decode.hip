@@ -60,7 +60,14 @@ struct DecParams {
 };
 
 
-template <class E, int D, bool ALIBI, bool MASK>
+template <bool NT, class T>
+__device__ __forceinline__ T load_once(const T* ptr) {
+  if constexpr (NT) return __builtin_nontemporal_load(ptr);
+  return *ptr;
+}
+
+// NT: K/V with non-temporal loads (decode_run_plan, host_plan.cpp).
+template <class E, int D, bool ALIBI, bool MASK, bool NT>
 __global__ __launch_bounds__(256) void attn_decode16(DecParams p) {
   constexpr int KK = D / 32;  // score MFMAs per 16-key step
   constexpr int VC = D / 16;  // consecutive d of one V row held by a lane
@@ -133,14 +140,14 @@ __global__ __launch_bounds__(256) void attn_decode16(DecParams p) {
     const int j = min(j0 + lr, klast);
     const uint16_t* krow = kbase + (int64_t)j * p.k_ss;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) kv[kk] = *(const u32x4_t*)(krow + kk * 32);
+    for (int kk = 0; kk < KK; ++kk) kv[kk] = load_once<NT>((const u32x4_t*)(krow + kk * 32));
   };
   // V: lane holds keys j0 + lg*4 + v (v = 0..3), d = lr*VC .. +VC.
   auto load_v = [&](int j0, VT (&vv)[4]) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int j = min(j0 + lg * 4 + v, klast);
-      vv[v] = *(const VT*)(vbase + (int64_t)j * p.v_ss);
+      vv[v] = load_once<NT>((const VT*)(vbase + (int64_t)j * p.v_ss));
     }
   };
 
@@ -357,20 +364,26 @@ __global__ __launch_bounds__(256) void attn_decode_combine(DecParams p) {
   if (p.lse && t == 0) p.lse[((int64_t)b * p.Hq + hq) * p.Sq + i] = (mm + __log2f(LL)) * kLn2;
 }
 
-template <class E, int D>
+template <class E, int D, bool NT>
 hipError_t launch_decode(const DecParams& p, int feat, hipStream_t st) {
   const dim3 grid((unsigned)((int64_t)p.B * p.Hkv * p.RG * p.n_splits)), block(256);
   hipError_t err;
   switch (feat) {
-    case 0: err = launch_kernel(&attn_decode16<E, D, false, false>, grid, block, 0, st, p); break;
-    case kFeatAlibi: err = launch_kernel(&attn_decode16<E, D, true, false>, grid, block, 0, st, p); break;
-    case kFeatMask: err = launch_kernel(&attn_decode16<E, D, false, true>, grid, block, 0, st, p); break;
-    case kFeatAlibi | kFeatMask: err = launch_kernel(&attn_decode16<E, D, true, true>, grid, block, 0, st, p); break;
+    case 0: err = launch_kernel(&attn_decode16<E, D, false, false, NT>, grid, block, 0, st, p); break;
+    case kFeatAlibi: err = launch_kernel(&attn_decode16<E, D, true, false, NT>, grid, block, 0, st, p); break;
+    case kFeatMask: err = launch_kernel(&attn_decode16<E, D, false, true, NT>, grid, block, 0, st, p); break;
+    case kFeatAlibi | kFeatMask: err = launch_kernel(&attn_decode16<E, D, true, true, NT>, grid, block, 0, st, p); break;
     default: return hipErrorNotSupported;
   }
   if (err != hipSuccess || p.n_splits == 1) return err;
   const int64_t rows = (int64_t)p.B * p.Hkv * p.M;
   return launch_kernel(&attn_decode_combine<E, D>, dim3((unsigned)rows), dim3(256), 0, st, p);
+}
+template <class E, int D>
+hipError_t launch_decode(const DecParams& p, bool streamed, int feat, hipStream_t st) {
+  if constexpr (D == 128)
+    if (streamed) return launch_decode<E, D, true>(p, feat, st);
+  return launch_decode<E, D, false>(p, feat, st);
 }
 
 }  // namespace trinix
@@ -397,7 +410,9 @@ namespace {
 
 // Launches the split-KV forward of a validated call with plan `pl`; the
 // partial results go to `workspace` (pl.ws_bytes bytes, 16-byte aligned).
-int launch_splitkv(const trinix_attn_fwd_args* a, const SplitPlan& pl, void* workspace, hipStream_t st) {
+int launch_splitkv(const trinix_attn_fwd_args* a, SplitPlan pl, void* workspace, hipStream_t st) {
+  bool streamed;
+  decode_run_plan(a, &pl, &streamed);
   DecParams p;
   p.q = (const uint16_t*)a->q;
   p.k = (const uint16_t*)a->k;
@@ -438,9 +453,11 @@ int launch_splitkv(const trinix_attn_fwd_args* a, const SplitPlan& pl, void* wor
 
   hipError_t err;
   if (a->dtype == TRINIX_BF16)
-    err = a->head_dim == 128 ? launch_decode<BF16, 128>(p, feat, st) : launch_decode<BF16, 64>(p, feat, st);
+    err = a->head_dim == 128 ? launch_decode<BF16, 128>(p, streamed, feat, st)
+                             : launch_decode<BF16, 64>(p, streamed, feat, st);
   else
-    err = a->head_dim == 128 ? launch_decode<F16, 128>(p, feat, st) : launch_decode<F16, 64>(p, feat, st);
+    err = a->head_dim == 128 ? launch_decode<F16, 128>(p, streamed, feat, st)
+                             : launch_decode<F16, 64>(p, streamed, feat, st);
   return err == hipSuccess ? TRINIX_OK : TRINIX_ERR_LAUNCH;
 }
 

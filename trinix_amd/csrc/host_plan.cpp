@@ -484,4 +484,55 @@ bool make_split_plan(const trinix_attn_fwd_args* a, SplitPlan* pl) {
   return true;
 }
 
+// The plan bounds the chunks (and fixes the workspace) at four workgroups per
+// CU; a launch runs the count among one to four workgroups per CU that costs
+// least.  A decode step is bound by HBM, and one workgroup on every CU already
+// saturates it: more only add chunks to merge and spread the reads.  Cost: the
+// read at 5.5 TB/s, times how unevenly whole workgroups fall on the CUs (a
+// workgroup alone on its CU in a partial grid reads up to 1 / 0.82 of its
+// share), 6% for more than one per CU, and 3 us for the merge.  Head_dim 64
+// (half the bytes per load) follows no such rule: one workgroup per CU where
+// that fills them, the plan's count otherwise (B=12 S=3000 16 heads: 1152
+// workgroups 34.8 us, 768 37.5, 192 39.6).
+// Measured, bf16, 8 KV heads of D=128 unless noted, caches cold, graph-timed,
+// us as planned | run: B=16 S=8192 113.7 | 99.9 (256 workgroups, non-temporal),
+// B=4 S=8000 36.4 | 30.6, B=24 S=4000 84.6 | 78.2 (192), B=48 S=2000 ceil-planned
+// 1152 86.3 | 81.6 (768), B=64 S=2000 104.6 | 98.2 (512, unsplit), B=16 S=1000
+// 23.4 | 19.1, B=16 S=3000 16 heads of D=64 47.4 | 37.9.
+// Non-temporal K/V loads pay where the workgroups fill the CUs evenly (B=16
+// S=8192 107.8 | 99.9 us, B=32 S=8000 193 | 189) and lose where CUs idle in the
+// last round (192 workgroups 78.2 | 88.3, 384 90.9 | 94.2, 128 9.8 | 10.1) and at
+// head_dim 64 (B=16 S=3000 16 heads 39.6 | 44.2); with several row groups the
+// K/V are read again, from L2.
+void decode_run_plan(const trinix_attn_fwd_args* a, SplitPlan* pl, bool* streamed) {
+  const int64_t items = a->batch * a->nheads_kv * pl->RG, span = (int64_t)pl->khi - pl->klo;
+  auto rounds = [&](int64_t n) { return (items * n + kSmallGrid - 1) / kSmallGrid; };
+  auto uneven = [&](int64_t n) { return (double)(rounds(n) * kSmallGrid) / (double)(items * n); };
+  auto run = [&](int64_t n, int64_t* chunk) {  // chunks of whole 64 keys, as planned
+    *chunk = ((span + n - 1) / n + 63) / 64 * 64;
+    return (span + *chunk - 1) / *chunk;
+  };
+  if (pl->n_splits > 1 && !getenv("TRINIX_SPLITKV_CFG")) {
+    const double read_us = 4.0 * items * span * a->head_dim / 5.5e6;
+    double best = 1e30;
+    int64_t best_n = pl->n_splits;
+    for (int k = 1; k <= 4; ++k) {
+      int64_t n = std::min<int64_t>(pl->n_splits, kSmallGrid * k / items), chunk;
+      if (n < 1) continue;
+      n = run(n, &chunk);
+      if (a->head_dim == 64 && (k > 1 || uneven(n) > 1.07)) break;
+      const double share = rounds(n) > 1 ? 1.06 * uneven(n) : std::max(1.0, 0.82 * uneven(n));
+      const double us = read_us * share + (n > 1 ? 3.0 : 0.0);
+      if (us < best) {
+        best = us;
+        best_n = n;
+      }
+    }
+    int64_t chunk;
+    pl->n_splits = (int)run(best_n, &chunk);
+    pl->chunk = (int)chunk;
+  }
+  *streamed = a->head_dim == 128 && pl->RG == 1 && uneven(pl->n_splits) <= 1.07;
+}
+
 }  // namespace trinix

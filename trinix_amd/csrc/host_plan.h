@@ -100,5 +100,8 @@ struct SplitPlan {
 };
 // false if the split-KV kernel does not apply (then trinix_attn_fwd is the path).
 bool make_split_plan(const trinix_attn_fwd_args* a, SplitPlan* pl);
+// Lowers n_splits (and raises chunk) of a plan to what a launch runs, inside
+// the planned workspace; *streamed: K/V with non-temporal loads.
+void decode_run_plan(const trinix_attn_fwd_args* a, SplitPlan* pl, bool* streamed);
 
 }  // namespace trinix
