@@ -88,9 +88,9 @@ static bool wide_grid(int64_t batch, int64_t hq, int64_t sq, bool banded) {
 //     35.3, 192 x 32 40.4 | 41.0; full rows 96 x 24 31.2 | 25.8, 240 x 24 35.6 |
 //     34.1; ALiBi 256 x 32 47.2 | 41.9; where it loses: 32 x 2 7.7 | 8.0, 128 x 3
 //     8.4 | 8.8, 256 x 8 16.6 | 17.2, 384 x 16 27.9 | 30.2, 512 x 32 49.9 | 52.0
-//   D=256 48 x 11 30.0 | 25.8, 128 x 32 76.7 | 61.1, 128 x 7 windowed 27.7 | 22.9,
-//     full rows 128 x 16 49.2 | 41.5; loses: 128 x 3 14.2 | 15.2, 192 x 8 29.4 |
-//     33.1, 192 x 24 full 69.4 | 97.9
+//   D=256 48 x 11 31.3 | 27.0, 128 x 32 76.7 | 60.0, full rows 128 x 16 44.6 |
+//     36.7; loses: 128 x 3 14.2 | 15.2, 192 x 8 27.8 | 31.8, 192 x 24 full 62.7 |
+//     85.5, 192 x 32 75.2 | 81.5
 static bool key_split(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, int64_t chain) {
   if (head_dim < 128 || chain < 4 || batch * hq > kSmallGrid) return false;
   const int64_t wgs = batch * hq * ((sq + 127) / 128);
