@@ -93,3 +93,16 @@ def test_padded_heads_with_dropout_and_mask(monkeypatch, keep_map):
     want = _run(triton_attn_func, [t.requires_grad_(True) for t in pad[:3]], pad[3], **kw)
     for a, b in zip(got, want):
         assert torch.equal(a, b[..., :D])
+
+
+@pytest.mark.parametrize("D", [80, 100])
+def test_padded_heads_output_written_before_the_backward(D):
+    """The backward reads its own copy of the output: scaling the returned one
+    in place scales the gradients alone (by a power of two, bitwise)."""
+    ts = [t.to(DEV) for t in _tensors(2, 70, 90, 3, 3, D, torch.float16, 8)]
+    leaves = [t.requires_grad_(True) for t in ts[:3]]
+    for _ in range(2):  # the second from the layout's launch templates
+        want = torch.autograd.grad(triton_attn_func(*leaves), leaves, ts[3])
+        got = torch.autograd.grad(triton_attn_func(*leaves).mul_(0.5), leaves, ts[3] * 2)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)

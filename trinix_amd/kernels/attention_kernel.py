@@ -439,7 +439,7 @@ def _train_cached(tkey, q, k, v):
         nat.check(lib.trinix_attn_fwd_narrow(ctypes.byref(a), D, stream), "trinix_attn_fwd_narrow")
     state = dict(q=q, k=k, v=v, out=out, lse=lse, D=D, d_kernel=int(a.head_dim), narrow=ent.pad is not None, args=a,
                  launch=ent, dropout=(float(a.dropout_p), int(a.dropout_seed), 0), dropout_state=None, keep_map=keep_map)
-    return out, lse, state
+    return (out if ent.pad is None else out.clone()), lse, state
 
 
 def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_slopes, rotary_cos, rotary_sin,
@@ -709,6 +709,8 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
                      dropout_state=drop_state, keep_map=keep_map)
     if d_kernel != D and not narrow:
         out = out[..., :D].contiguous()
+    elif narrow and keep_state:
+        out = out.clone()  # the caller may write to its output before the backward, which reads the state's
     return out, lse, state
 
 
