@@ -117,6 +117,29 @@ static void check_plan(const trinix_attn_fwd_args& a, const SplitPlan& pl) {
   CHECK(pl.ws_bytes == (pl.n_splits > 1 ? rows * pl.n_splits * (a.head_dim + 1) * 4 : 0), "plan workspace");
 }
 
+// Grids of a backward plan, in 128 bits.  The fp32 and head_dim 256 kernels
+// refuse what blocks of 32 keys or rows, or of 4 rows in the delta pass,
+// cannot cover in one grid; the others what their own blocks cannot.
+static void check_bwd_grids(const trinix_attn_bwd_args& a, int rc, const BwdPlan& pl, bool generic) {
+  typedef __int128 wide;
+  const wide lim = (wide)1 << 31, bq = (wide)a.batch * a.nheads_q, bkv = (wide)a.batch * a.nheads_kv;
+  const int64_t delta_rows = a.dtype == TRINIX_F32 ? 1024 / a.head_dim : 2048 / a.head_dim;  // per workgroup
+  const wide delta = (bq * a.seqlen_q + delta_rows - 1) / delta_rows;
+  const bool fits32 = bkv * ((a.seqlen_k + 31) / 32) < lim && bq * ((a.seqlen_q + 31) / 32) < lim &&
+                       (bq * a.seqlen_q + 3) / 4 < lim;
+  CHECK(rc == TRINIX_OK || rc == TRINIX_ERR_BAD_SHAPE, "bwd plan status %d", rc);
+  // (at most four workgroups of different columns share a block of 128 or 64)
+  const bool one_each = bkv * ((a.seqlen_k + 63) / 64) * 4 < lim && bq * ((a.seqlen_q + 63) / 64) * 2 < lim;
+  if (generic) CHECK(rc == TRINIX_OK ? fits32 : !fits32 || !one_each, "fp32 / head_dim 256 plan: rc %d", rc);
+  if (rc != TRINIX_OK) return;
+  CHECK(delta < lim, "delta grid");
+  CHECK(bkv * pl.num_kblk * pl.kv_hs < lim && bq * pl.num_mblk * pl.dq_hs < lim, "gradient grids");
+  const int bk = 128 / pl.kv_ks, bm = pl.dq_wide ? 256 : 128 / pl.dq_ks;
+  CHECK((wide)pl.num_kblk * bk >= a.seqlen_k && (wide)pl.num_mblk * bm >= a.seqlen_q, "blocks cover");
+  if (pl.kv_T) CHECK(bkv * pl.kv_P < lim && bkv * pl.num_kblk * 16 < lim, "piece grids");
+  CHECK((wide)pl.ws_bytes == (pl.kv_T ? bkv * pl.kv_P * 2 * 128 * a.head_dim * 4 : 0), "piece workspace");
+}
+
 int main() {
   int cases = 0;
   // ---- status codes of the forward's validation
@@ -194,6 +217,29 @@ int main() {
     set_mask(a, 0, 0, 70000, 1);
     CHECK(validate_bwd_args(&a) == TRINIX_OK, "bwd contiguous mask of 70000^2");
     cases += 9;
+  }
+  // ---- the backward plan's grids: a launch has fewer than 2^31 workgroups,
+  // whatever the arguments that validation accepts (their products pass 2^63)
+  {
+    const int64_t big = (1 << 20) - 1, longest = (1ll << 30) - 1;
+    const int64_t sizes[][5] = {{big, longest, longest, big, big}, {big, 1, longest, big, 1}, {big, longest, 1, big, big},
+                                {1 << 19, longest, longest, 1 << 19, 1 << 19}, {1, longest, longest, big, 1},
+                                {1, 1 << 17, 1 << 17, big, 1}, {16, 1 << 24, 1 << 24, 128, 128},
+                                {1, 1 << 25, 1 << 25, 256, 256}, {1, longest, longest, 1, 1}};
+    for (const auto& z : sizes)
+      for (int dtype : {TRINIX_F32, TRINIX_F16, TRINIX_BF16})
+        for (int64_t D : {64, 128, 256})
+          for (bool split : {false, true}) {
+            trinix_attn_bwd_args a = valid_bwd();
+            a.batch = z[0], a.seqlen_q = z[1], a.seqlen_k = z[2], a.nheads_q = z[3], a.nheads_kv = z[4];
+            a.dtype = dtype, a.head_dim = D;
+            CHECK(validate_bwd_args(&a) == TRINIX_OK, "bwd sizes accepted");
+            BwdPlan pl;
+            const int rc = plan_bwd(&a, &pl, split);
+            const bool generic = dtype == TRINIX_F32 || D == 256;
+            check_bwd_grids(a, rc, pl, generic);
+            ++cases;
+          }
   }
   // ---- the tuning override TRINIX_ATTN_CFG="nw,occ,bn[,ks]": ks 0 (the
   // per-item split), 1 and 2 are taken, anything else leaves the planner's
@@ -295,6 +341,9 @@ int main() {
       CHECK((__int128)rows * a.mask_stride[2] < ((__int128)1 << 31), "sub-tile row offsets fit 31 bits");
       CHECK((__int128)(a.seqlen_k - 1) * a.mask_stride[3] < ((__int128)1 << 31), "key offsets fit 31 bits");
     }
+    BwdPlan bp;
+    const int prc = plan_bwd(&a, &bp, next_u64() % 2 == 0);
+    check_bwd_grids(a, prc, bp, a.dtype == TRINIX_F32 || a.head_dim == 256);
     const bool masked = next_u64() % 2 == 0;
     if (pick_dq_wide(a.head_dim, a.batch, a.nheads_q, a.seqlen_q, a.causal || a.has_window, masked))
       CHECK(a.head_dim == 128 && !masked, "wide dQ only at head_dim 128 without a mask");

@@ -385,6 +385,13 @@ static void plan_bwd_pieces(const trinix_attn_bwd_args* a, BwdPlan* pl) {
   if (pl->kv_T) pl->ws_bytes = groups * pl->kv_P * 2 * BK * (int64_t)D * 4;
 }
 
+// Workgroups of a launch of `blocks` per (batch, head), or -1 where no grid
+// holds them (2^31); batch, heads < 2^20, 0 < blocks < 2^32.
+static int64_t grid_of(int64_t batch, int64_t heads, int64_t blocks) {
+  const int64_t bh = batch * heads;
+  return bh < (1ll << 31) && bh * blocks < (1ll << 31) ? bh * blocks : -1;
+}
+
 int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl, bool split) {
   const bool f32 = a->dtype == TRINIX_F32;
   const int64_t D = a->head_dim;
@@ -392,6 +399,16 @@ int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl, bool split) {
   pl->dq_wide = !pl->generic && pick_dq_wide(D, a->batch, a->nheads_q, a->seqlen_q, a->causal || a->has_window,
                                              a->mask != nullptr);
   pl->dq_ks = pl->kv_ks = pl->dq_hs = pl->kv_hs = 1;
+  // Every grid is bounded before a plan is chosen from its size.  The fp32 and
+  // head_dim 256 calls take what blocks of 32 rows and keys, and 4 rows of the
+  // delta pass, can cover; the others 128 keys, 128 or 256 rows, and the
+  // 2048 / D rows of a delta workgroup.
+  const int64_t bq = pl->generic ? 32 : (pl->dq_wide ? 256 : 128), bk0 = pl->generic ? 32 : 128;
+  const int64_t bd = pl->generic ? 4 : 2048 / D;
+  if (grid_of(a->batch, a->nheads_q, (a->seqlen_q + bq - 1) / bq) < 0 ||
+      grid_of(a->batch, a->nheads_kv, (a->seqlen_k + bk0 - 1) / bk0) < 0 ||
+      (a->batch * a->nheads_q * a->seqlen_q + bd - 1) / bd >= (1ll << 31))  // < 2^31 * 256 rows here
+    return TRINIX_ERR_BAD_SHAPE;
   if (pl->generic) {
     if (D == 256) {  // column splits: the kernels' registers
       pl->kv_hs = f32 ? 4 : 2;
@@ -412,25 +429,31 @@ int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl, bool split) {
   const int bm = pl->dq_wide ? 256 : 128 / pl->dq_ks, bk = 128 / pl->kv_ks;
   pl->num_kblk = (int)((a->seqlen_k + bk - 1) / bk);
   pl->num_mblk = (int)((a->seqlen_q + bm - 1) / bm);
-  if (a->batch * a->nheads_q * pl->num_mblk * pl->dq_hs >= (1ll << 31) ||
-      a->batch * a->nheads_kv * pl->num_kblk * pl->kv_hs >= (1ll << 31))
+  if (grid_of(a->batch, a->nheads_q, (int64_t)pl->num_mblk * pl->dq_hs) < 0 ||
+      grid_of(a->batch, a->nheads_kv, (int64_t)pl->num_kblk * pl->kv_hs) < 0)
     return TRINIX_ERR_BAD_SHAPE;
   pl->kv_T = pl->kv_P = 0;
   pl->ws_bytes = 0;
+  // items of a key block (query tiles of a group's q-heads) count in 31 bits
+  const int64_t G = a->nheads_q / a->nheads_kv;
+  const bool countable = G * ((a->seqlen_q + 63) / 64) < (1ll << 31);
   if (split && !pl->generic) {
     if (const char* env = getenv("TRINIX_BWD_PIECES")) {  // pieces of at most this many items, 0: whole (tuning and tests)
       const int T = atoi(env);
-      if (T > 0 && pl->num_kblk <= kMaxSplitKblk) {
+      if (T > 0 && pl->num_kblk <= kMaxSplitKblk && countable) {
         int dlo, dhi;
         band_offsets(a->causal != 0, a->has_window != 0, clamp_window(a->window_left), clamp_window(a->window_right), dlo,
                      dhi);
+        int64_t pieces = 0;
         for (int k = 0; k < pl->num_kblk; ++k)
-          pl->kv_P += bwd_pieces(bwd_kv_items(k, 128, (int)(a->nheads_q / a->nheads_kv), (int)a->seqlen_q,
-                                              (int)a->seqlen_k, dlo, dhi, 64), T);
-        pl->kv_T = T;
-        pl->ws_bytes = a->batch * a->nheads_kv * pl->kv_P * 2 * 128 * D * 4;
+          pieces += bwd_pieces(bwd_kv_items(k, 128, (int)G, (int)a->seqlen_q, (int)a->seqlen_k, dlo, dhi, 64), T);
+        if (grid_of(a->batch, a->nheads_kv, pieces) >= 0 && grid_of(a->batch, a->nheads_kv, 16 * pl->num_kblk) >= 0) {
+          pl->kv_T = T;
+          pl->kv_P = (int)pieces;
+          pl->ws_bytes = a->batch * a->nheads_kv * pieces * 2 * 128 * D * 4;
+        }
       }
-    } else {
+    } else if (countable) {
       plan_bwd_pieces(a, pl);
     }
   }
