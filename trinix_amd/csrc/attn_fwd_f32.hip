@@ -121,11 +121,15 @@ __global__ __launch_bounds__(256, OCC) void attn_fwd_f32(const FwdParams p) {
       m_run = m_new;
     }
     const float m_use = m_run == -INFINITY ? 0.f : m_run;  // all keys so far masked: exp2(-inf - 0) = 0
+    // summed within the tile first: a running sum over the keys would round
+    // once per key of the row instead of once per tile
+    float sum = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       x[v] = __builtin_amdgcn_exp2f(x[v] - m_use);
-      l_run += x[v];
+      sum += x[v];
     }
+    l_run += sum;
     if (p.use_dropout) {
 #pragma unroll
       for (int vp = 0; vp < 2; ++vp) {  // 8-key groups vq = 2vp, 2vp + 1
