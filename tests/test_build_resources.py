@@ -87,3 +87,21 @@ def test_shipped_kernels_do_not_spill():
     assert len([n for _, n, _ in rows if "attn_fwd_mfma16" in n]) >= 2 * 3 * 8
     for src, name, f in rows:
         assert f["scratch"] == "0" and f["vgpr_spill"] == "0" and f["asm_spill_annotations"] == "0", (src, name, f)
+
+
+def test_whole_block_kernels_carry_no_piece_or_narrow_code():
+    """The piece map and the narrow output rows are template flags: as run-time
+    values of one kernel they raised the scalar-register spills of every call
+    (dK/dV at head_dim 128 2 -> 7, with the keep map 20 -> 35; at head_dim 64
+    7 -> 16 and 22 -> 37; the masked keep-map forward 35 -> 53) and cost the
+    whole-block backward 1%.  The limits are the counts without that code."""
+    spills = {name: int(f["sgpr_spill"]) for _, name, f in _report_rows()}
+    for dt in ("4BF16", "3F16"):
+        dkdv = "attn_bwd_dkdvINS_{}ELi{}ELb0ELb0ELi{}ELb{}E"
+        for D, drop, limit in ((128, 0, 2), (128, 2, 20), (64, 0, 7), (64, 2, 22)):
+            whole, ext = ([n for n in spills if dkdv.format(dt, D, drop, e) in n] for e in (0, 1))
+            assert len(whole) == len(ext) == 1, (dt, D, drop)
+            assert spills[whole[0]] <= limit, (whole, spills[whole[0]])
+        # head_dim 64, two wavefronts per row group, mask and keep map
+        fwd = [n for n in spills if f"attn_fwd_mfma16INS_{dt}ELi64ELi64ELi4ELi2ELi2ELb0ELb1ELi2ELb0ELb0E" in n]
+        assert len(fwd) == 1 and spills[fwd[0]] <= 35, (fwd, spills.get(fwd[0] if fwd else None))

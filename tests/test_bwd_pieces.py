@@ -99,3 +99,69 @@ def test_pieces_match_whole_blocks(monkeypatch, case, dtype, T):
         assert torch.equal(a, b), name
         d, scale = (a.double() - w.double()).abs(), w.double().abs().max()
         assert (d <= 2 * u * w.double().abs() + 1e-5 * scale).all(), (name, d.max().item(), scale.item())
+
+
+
+FEATURES = [
+    # (B, Sq, Sk, Hq, Hkv, D, kwargs): the mask and ALiBi variants of the kernel, and head_dims between the kernels'
+    # (narrow rows, the partial sums behind a padded dout)
+    (2, 150, 260, 4, 2, 64, dict(attn_mask=True)),
+    (1, 260, 260, 4, 1, 128, dict(attn_mask=True, alibi_slopes=True)),
+    (2, 130, 200, 4, 2, 64, dict(alibi_slopes=True, causal=True)),
+    (1, 140, 270, 4, 2, 128, dict(attn_mask=True, dropout_p=0.25)),
+    (1, 140, 140, 2, 1, 64, dict(attn_mask=True, alibi_slopes=True, dropout_p=0.25, causal=True)),
+    (2, 150, 260, 4, 2, 40, dict(causal=True)),
+    (1, 260, 150, 4, 1, 80, dict()),
+    (2, 150, 260, 4, 2, 72, dict(attn_mask=True, alibi_slopes=True)),
+    (1, 140, 270, 4, 2, 112, dict(dropout_p=0.25, causal=True)),
+    (1, 140, 270, 4, 2, 56, dict(attn_mask=True, dropout_p=0.25)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [0, 1, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", range(len(FEATURES)))
+def test_features_in_pieces(monkeypatch, case, dtype, T):
+    """Whole blocks (T = 0) and pieces against float64 autograd: twice the eager
+    error plus 2e-3 of the scale, the bar of the other gradient tests; with
+    dropout, pieces against whole blocks of the same seed alone (bound as in
+    test_pieces_match_whole_blocks)."""
+    B, Sq, Sk, Hq, Hkv, D, kw = FEATURES[case]
+    print(f"pieces {FEATURES[case]} {dtype} T {T}", flush=True)
+    g = torch.Generator().manual_seed(100 + case)
+    ts = [torch.randn(s, generator=g).to(dtype)
+          for s in ((B, Sq, Hq, D), (B, Sk, Hkv, D), (B, Sk, Hkv, D), (B, Sq, Hq, D))]
+    kw = dict(kw)
+    if "attn_mask" in kw:  # a block mask: some 64-key blocks are skipped, key block 0 stays open
+        m = torch.zeros(Sq, Sk)
+        m[: Sq // 2, 64:128] = float("-inf")
+        m[Sq // 2:, 192:] = -1.5
+        kw["attn_mask"] = m
+    if "alibi_slopes" in kw:
+        kw["alibi_slopes"] = orc.alibi_slopes(Hq)
+    gpu = {k: v.to(DEV) if torch.is_tensor(v) else v for k, v in kw.items()}
+
+    def grads(pieces):
+        monkeypatch.setenv("TRINIX_BWD_PIECES", str(pieces))
+        monkeypatch.setattr(ak, "_TRAIN_LAUNCHES", {})
+        torch.manual_seed(77)
+        leaves = [t.to(DEV).requires_grad_(True) for t in ts[:3]]
+        return [t.cpu().double() for t in torch.autograd.grad(triton_attn_func(*leaves, **gpu), leaves, ts[3].to(DEV))]
+
+    got = grads(T)
+    if "dropout_p" in kw:
+        u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        for name, w, a in zip(("dq", "dk", "dv"), grads(0), got):
+            d, scale = (a - w).abs(), w.abs().max()
+            assert (d <= 2 * u * w.abs() + 1e-5 * scale).all(), (name, d.max().item(), scale.item())
+        return
+
+    def ref(dt):
+        leaves = [t.to(dt).requires_grad_(True) for t in ts[:3]]
+        return [t.double() for t in torch.autograd.grad(orc.functional_attention(*leaves, **kw), leaves, ts[3].to(dt))]
+
+    for name, h, e, t in zip(("dq", "dk", "dv"), got, ref(dtype), ref(torch.float64)):
+        scale = t.abs().max().item()
+        err_h, err_e = (h - t).abs().max().item(), (e - t).abs().max().item()
+        assert err_h <= 2 * err_e + 2e-3 * scale, (name, err_h, err_e, scale)

@@ -210,14 +210,20 @@ int run_bwd(const trinix_attn_bwd_args* a, int64_t d_out, void* workspace, int64
   if (a->head_dim == 256) {
     err = bf ? launch_delta<BF16, 256>(p, st) : launch_delta<F16, 256>(p, st);
     if (err == hipSuccess) err = bf ? launch_bwd_generic_bf16(p, plan, st) : launch_bwd_generic_f16(p, plan, st);
-  } else if (a->head_dim == 128) {
-    err = bf ? launch_delta<BF16, 128>(p, st) : launch_delta<F16, 128>(p, st);
-    use_padded_dout(p, 128);
-    if (err == hipSuccess) err = bf ? launch_bwd16_bf16_d128(p, feat, st) : launch_bwd16_f16_d128(p, feat, st);
   } else {
-    err = bf ? launch_delta<BF16, 64>(p, st) : launch_delta<F16, 64>(p, st);
-    use_padded_dout(p, 64);
-    if (err == hipSuccess) err = bf ? launch_bwd16_bf16_d64(p, feat, st) : launch_bwd16_f16_d64(p, feat, st);
+    const bool d128 = a->head_dim == 128;
+    if (d128) err = bf ? launch_delta<BF16, 128>(p, st) : launch_delta<F16, 128>(p, st);
+    else err = bf ? launch_delta<BF16, 64>(p, st) : launch_delta<F16, 64>(p, st);
+    use_padded_dout(p, (int)a->head_dim);
+    LaunchBwd16* dkdv = d128 ? (bf ? launch_dkdv16_bf16_d128 : launch_dkdv16_f16_d128)
+                             : (bf ? launch_dkdv16_bf16_d64 : launch_dkdv16_f16_d64);
+    if (p.kv_T || d_out < a->head_dim)
+      dkdv = d128 ? (bf ? launch_dkdv16x_bf16_d128 : launch_dkdv16x_f16_d128)
+                  : (bf ? launch_dkdv16x_bf16_d64 : launch_dkdv16x_f16_d64);
+    LaunchBwd16* dq = d128 ? (bf ? launch_dq16_bf16_d128 : launch_dq16_f16_d128)
+                           : (bf ? launch_dq16_bf16_d64 : launch_dq16_f16_d64);
+    if (err == hipSuccess) err = dkdv(p, feat, st);
+    if (err == hipSuccess) err = dq(p, feat, st);
   }
   return err == hipSuccess ? TRINIX_OK : TRINIX_ERR_LAUNCH;
 }

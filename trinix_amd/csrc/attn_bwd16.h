@@ -292,7 +292,12 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce(const BwdParams p) {
   *(u32x2_t*)(row + d0) = (u32x2_t){E::pack(s[0] * f, s[1] * f), E::pack(s[2] * f, s[3] * f)};
 }
 
-template <class E, int D, bool ALIBI, bool MASK, int DROP>
+// EXT: pieces (p.kv_T) or narrow output rows (p.d_out < D); the other calls
+// keep a kernel without either.  As run-time values of one kernel they cost
+// the whole-block calls 5..19 SGPR spills and 1%: S=8192 32/8 heads D=128,
+// forward + backward, same-box pairs without them | with, 2252 | 2271 us;
+// without them | with this flag 2313 | 2311, 2366 | 2358.
+template <class E, int D, bool ALIBI, bool MASK, int DROP, bool EXT>
 __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
   DropKey dkey{};
   if constexpr (DROP) dkey = drop_key(p);
@@ -319,7 +324,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
   const Band band(p);
   // (index_map.h) key block, and which of its pieces (one unless kv_T cuts it)
   int kblk, hkv, b, np = 1, pk = 0, slot = 0;
-  if (p.kv_T == 0) {
+  if (!EXT || p.kv_T == 0) {
     const KvItem wi = bwd_kv_item((int)blockIdx.x, p.B, p.Hkv, p.num_kblk, p.causal != 0);
     kblk = wi.kblk, hkv = wi.hkv, b = wi.b;
   } else {
@@ -342,9 +347,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
   bwd_query_tiles(kb0, BK, p.Sq, p.Sk, band.dlo, band.dhi, BQ, qt_lo, qt_hi);
   const int nqt = qt_hi - qt_lo;
   // item = (q-head of the group, query tile); this workgroup's run of them
-  const int all_items = nqt > 0 ? p.G * nqt : 0, it0 = bwd_piece_first(all_items, np, pk);
-  const int n_items = bwd_piece_first(all_items, np, pk + 1) - it0;
-  const int gh0 = nqt > 0 ? it0 / nqt : 0, qt0 = nqt > 0 ? qt_lo + it0 % nqt : qt_lo;
+  int n_items = nqt > 0 ? p.G * nqt : 0, gh0 = 0, qt0 = qt_lo;
+  if constexpr (EXT) {
+    const int it0 = bwd_piece_first(n_items, np, pk);
+    n_items = bwd_piece_first(n_items, np, pk + 1) - it0;
+    if (nqt > 0) gh0 = it0 / nqt, qt0 = qt_lo + it0 % nqt;
+  }
 
   // ---- tile copies: Q and dO rows (16-byte units, swizzled), lse and delta
   auto ld_row = [&](int l) __attribute__((always_inline)) { return tile_copy_row(wave, LPW, l, lane, UPR); };
@@ -687,7 +695,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
 
     // ---- epilogue: a piece's fp32 partial sums, in the order of the lanes
     // (bwd_dkdv_reduce adds them up)
-    if (np > 1) {
+    if (EXT && np > 1) {
       float* part = p.part + ((int64_t)slot * 2 + (SB ? 1 : 0)) * BK * D + (kg * DB * 4 * 64 + lane) * 4;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -709,7 +717,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq) {
           const int d0 = db * 32 + vq * 8 + g * 4;
-          if (d0 >= p.d_out) continue;  // columns of zero padding
+          if (EXT && d0 >= p.d_out) continue;  // columns of zero padding
           *(u32x2_t*)(row + d0) = (u32x2_t){E::pack(acc[db][vq * 4 + 0] * f, acc[db][vq * 4 + 1] * f),
                                             E::pack(acc[db][vq * 4 + 2] * f, acc[db][vq * 4 + 3] * f)};
         }
@@ -1017,65 +1025,59 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_bwd_dq(const BwdParams p) {
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
         const int d0 = db * 32 + vq * 8 + g * 4;
-        if (d0 >= p.d_out) continue;  // columns of zero padding
+        if (db * 32 + vq * 8 >= p.d_out) continue;  // columns of zero padding (whole groups of 8)
         *(u32x2_t*)(qrow + d0) = (u32x2_t){E::pack(acc[db][vq * 4 + 0] * f, acc[db][vq * 4 + 1] * f),
                                            E::pack(acc[db][vq * 4 + 2] * f, acc[db][vq * 4 + 3] * f)};
       }
   }
 }
 
-// Launch of both gradient kernels for one (dtype, D); feat = kFeatAlibi |
-// kFeatMask | kFeatDropout.
-// Launch of both gradient kernels of one feature set; DROP as in the
-// kernels (0 none, 1 regenerated keep mask, 2 the forward's keep map).
+// Launch of one feature set; DROP as in the kernels (0 none, 1 regenerated
+// keep mask, 2 the forward's keep map), EXT as in attn_bwd_dkdv.
+template <class E, int D, bool A, bool M, int DROP, bool EXT>
+hipError_t launch_bwd_dkdv(const BwdParams& p, hipStream_t st) {
+  const dim3 grid((unsigned)(p.B * p.Hkv * (p.kv_T ? p.kv_P : p.num_kblk)));
+  const hipError_t e = launch_kernel(&attn_bwd_dkdv<E, D, A, M, DROP, EXT>, grid, dim3(512), 0, st, p);
+  if constexpr (EXT)
+    if (e == hipSuccess && p.kv_T)
+      return launch_kernel(&bwd_dkdv_reduce<E, D, DROP != 0>, dim3((unsigned)(p.B * p.Hkv * p.num_kblk * (D / 32 * 4)), 2),
+                           dim3(256), 0, st, p);
+  return e;
+}
 template <class E, int D, bool A, bool M, int DROP>
-hipError_t launch_bwd_pair(const BwdParams& p, hipStream_t st) {
-  const dim3 g_kv((unsigned)(p.B * p.Hkv * (p.kv_T ? p.kv_P : p.num_kblk))), g_q((unsigned)(p.B * p.Hq * p.num_mblk)), blk(256),
-      blk_kv(512);
-  hipError_t e = launch_kernel(&attn_bwd_dkdv<E, D, A, M, DROP>, g_kv, blk_kv, 0, st, p);
-  if (e == hipSuccess && p.kv_T)
-    e = launch_kernel(&bwd_dkdv_reduce<E, D, DROP != 0>, dim3((unsigned)(p.B * p.Hkv * p.num_kblk * (D / 32 * 4)), 2), blk, 0,
-                      st, p);
-  if (e != hipSuccess) return e;
+hipError_t launch_bwd_dq(const BwdParams& p, hipStream_t st) {
+  const dim3 grid((unsigned)(p.B * p.Hq * p.num_mblk));
   if constexpr (D == 128 && !M)
-    if (p.dq_wide) return launch_kernel(&attn_bwd_dq<E, D, A, M, DROP, 8, 128>, g_q, blk_kv, 0, st, p);
-  return launch_kernel(&attn_bwd_dq<E, D, A, M, DROP, 4, 64>, g_q, blk, 0, st, p);
+    if (p.dq_wide) return launch_kernel(&attn_bwd_dq<E, D, A, M, DROP, 8, 128>, grid, dim3(512), 0, st, p);
+  return launch_kernel(&attn_bwd_dq<E, D, A, M, DROP, 4, 64>, grid, dim3(256), 0, st, p);
 }
 
-// Launch of both gradient kernels for one (dtype, D); feat = kFeatAlibi |
+// Launch of the dK/dV or the dQ kernel of one (dtype, D); feat = kFeatAlibi |
 // kFeatMask | kFeatDropout (with p.keep_map: the map-reading variants).
-template <class E, int D>
+enum class Bwd16 { kDkdv, kDkdvExt, kDq };
+template <class E, int D, Bwd16 W>
 hipError_t launch_bwd(const BwdParams& p, int feat, hipStream_t st) {
-  switch (feat & 7) {
-#define TRINIX_BWD_CASE(F)                                                                                \
-  case F:                                                                                                 \
-  {                                                                                                       \
-    constexpr bool A = (F & kFeatAlibi) != 0, M = (F & kFeatMask) != 0, DR = (F & kFeatDropout) != 0;     \
-    if constexpr (DR) {                                                                                   \
-      if (p.keep_map) return launch_bwd_pair<E, D, A, M, 2>(p, st);                                       \
-      return launch_bwd_pair<E, D, A, M, 1>(p, st);                                                       \
-    }                                                                                                     \
-    return launch_bwd_pair<E, D, A, M, 0>(p, st);                                                         \
-  }
-    TRINIX_BWD_CASE(0)
-    TRINIX_BWD_CASE(1)
-    TRINIX_BWD_CASE(2)
-    TRINIX_BWD_CASE(3)
-    TRINIX_BWD_CASE(4)
-    TRINIX_BWD_CASE(5)
-    TRINIX_BWD_CASE(6)
-    TRINIX_BWD_CASE(7)
-#undef TRINIX_BWD_CASE
-  }
-  return hipErrorNotSupported;
+  auto one = [&](auto a, auto m, auto drop) {
+    constexpr bool A = decltype(a)::value, M = decltype(m)::value;
+    constexpr int DR = decltype(drop)::value;
+    if constexpr (W == Bwd16::kDq) return launch_bwd_dq<E, D, A, M, DR>(p, st);
+    else return launch_bwd_dkdv<E, D, A, M, DR, W == Bwd16::kDkdvExt>(p, st);
+  };
+  auto drop = [&](auto a, auto m) {
+    if (!(feat & kFeatDropout)) return one(a, m, std::integral_constant<int, 0>{});
+    return p.keep_map ? one(a, m, std::integral_constant<int, 2>{}) : one(a, m, std::integral_constant<int, 1>{});
+  };
+  auto mask = [&](auto a) { return feat & kFeatMask ? drop(a, std::true_type{}) : drop(a, std::false_type{}); };
+  return feat & kFeatAlibi ? mask(std::true_type{}) : mask(std::false_type{});
 }
 
-#define TRINIX_ATTN_BWD16_LAUNCHER(NAME, E, D) \
-  hipError_t NAME(const BwdParams& p, int feat, hipStream_t st) { return launch_bwd<E, D>(p, feat, st); }
-
-hipError_t launch_bwd16_bf16_d64(const BwdParams& p, int feat, hipStream_t st);
-hipError_t launch_bwd16_bf16_d128(const BwdParams& p, int feat, hipStream_t st);
-hipError_t launch_bwd16_f16_d64(const BwdParams& p, int feat, hipStream_t st);
-hipError_t launch_bwd16_f16_d128(const BwdParams& p, int feat, hipStream_t st);
+// One function per (dtype, head_dim) and kernel, in translation units of
+// their own (launch_dkdv16x_*: dK/dV in pieces or with narrow rows).
+typedef hipError_t LaunchBwd16(const BwdParams& p, int feat, hipStream_t st);
+LaunchBwd16 launch_dkdv16_bf16_d64, launch_dkdv16_bf16_d128, launch_dkdv16_f16_d64, launch_dkdv16_f16_d128;
+LaunchBwd16 launch_dkdv16x_bf16_d64, launch_dkdv16x_bf16_d128, launch_dkdv16x_f16_d64, launch_dkdv16x_f16_d128;
+LaunchBwd16 launch_dq16_bf16_d64, launch_dq16_bf16_d128, launch_dq16_f16_d64, launch_dq16_f16_d128;
+#define TRINIX_ATTN_BWD16_LAUNCHER(NAME, E, D, WHICH) \
+  hipError_t NAME(const BwdParams& p, int feat, hipStream_t st) { return launch_bwd<E, D, Bwd16::WHICH>(p, feat, st); }
 
 }  // namespace trinix

@@ -3,5 +3,6 @@
 #include "attn_bwd16.h"
 
 namespace trinix {
-TRINIX_ATTN_BWD16_LAUNCHER(launch_bwd16_bf16_d128, BF16, 128)
+TRINIX_ATTN_BWD16_LAUNCHER(launch_dkdv16_bf16_d128, BF16, 128, kDkdv)
+TRINIX_ATTN_BWD16_LAUNCHER(launch_dq16_bf16_d128, BF16, 128, kDq)
 }  // namespace trinix

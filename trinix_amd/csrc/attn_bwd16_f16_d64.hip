@@ -3,5 +3,6 @@
 #include "attn_bwd16.h"
 
 namespace trinix {
-TRINIX_ATTN_BWD16_LAUNCHER(launch_bwd16_f16_d64, F16, 64)
+TRINIX_ATTN_BWD16_LAUNCHER(launch_dkdv16_f16_d64, F16, 64, kDkdv)
+TRINIX_ATTN_BWD16_LAUNCHER(launch_dq16_f16_d64, F16, 64, kDq)
 }  // namespace trinix

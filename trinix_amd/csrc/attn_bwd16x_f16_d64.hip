@@ -1,0 +1,7 @@
+// dK/dV kernels for f16, head_dim 64, in pieces or with narrow rows (one
+// translation unit per instantiation keeps compile times parallel).
+#include "attn_bwd16.h"
+
+namespace trinix {
+TRINIX_ATTN_BWD16_LAUNCHER(launch_dkdv16x_f16_d64, F16, 64, kDkdvExt)
+}  // namespace trinix

@@ -43,8 +43,11 @@
 namespace trinix {
 
 // DROP: 0 no dropout, 1 dropout, 2 dropout that also writes the keep map
-// (p.keep_map, index_map.h) for the backward.
-template <class E, int D, int BN, int NW, int OCC, int KS, bool ALIBI, bool MASK, int DROP, bool QN>
+// (p.keep_map, index_map.h) for the backward.  NARROW: p.d_out < D columns of
+// out are written (zero-padded q, k, v); with dropout a kernel of its own, as
+// the test alone takes the full-width one up to 18 SGPR spills, without
+// dropout a run-time test that costs no register.
+template <class E, int D, int BN, int NW, int OCC, int KS, bool ALIBI, bool MASK, int DROP, bool QN, bool NARROW>
 // The head_dim 64 mask kernels are held to three wavefronts per SIMD (168
 // VGPRs), except the one writing a keep map (it does not fit); the other
 // shapes to OCC.
@@ -746,7 +749,7 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
         const int d0 = db * 32 + vq * 8 + ge * 4;
-        if (d0 >= p.d_out) continue;  // columns of zero padding
+        if ((NARROW || !DROP) && db * 32 + vq * 8 >= p.d_out) continue;  // zero padding (whole groups of 8)
         const u32x2_t w2 = {E::pack(acc[db][vq * 4 + 0] * inv, acc[db][vq * 4 + 1] * inv),
                             E::pack(acc[db][vq * 4 + 2] * inv, acc[db][vq * 4 + 3] * inv)};
         *(u32x2_t*)(orow + d0) = w2;
@@ -759,13 +762,15 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
 template <class E, int D, int BN, int NW, int OCC, int KS>
 hipError_t launch_feat(const FwdParams& p, int feat, hipStream_t st) {
   const dim3 grid((unsigned)p.total_work), block(NW * 64);
-  switch (feat) {
+#define TRINIX_KERNEL(F, N)                                                                                     \
+  attn_fwd_mfma16<E, D, BN, NW, OCC, KS, (F & kFeatAlibi) != 0, (F & kFeatMask) != 0,                          \
+                  (F & kFeatKeepMap) ? 2 : ((F & kFeatDropout) ? 1 : 0), (F & kFeatQNorm) != 0, N>
 #define TRINIX_CASE(F)                                                                                          \
   case F:                                                                                                       \
-    return launch_kernel(&attn_fwd_mfma16<E, D, BN, NW, OCC, KS, (F & kFeatAlibi) != 0, (F & kFeatMask) != 0,  \
-                                          (F & kFeatKeepMap) ? 2 : ((F & kFeatDropout) ? 1 : 0),               \
-                                          (F & kFeatQNorm) != 0>,                                              \
-                         grid, block, 0, st, p);
+    if constexpr (((F) & kFeatDropout) && D <= 128)                                                             \
+      if (p.d_out < D) return launch_kernel(&TRINIX_KERNEL(F, true), grid, block, 0, st, p);                   \
+    return launch_kernel(&TRINIX_KERNEL(F, false), grid, block, 0, st, p);
+  switch (feat) {
     TRINIX_CASE(0)
     TRINIX_CASE(1)
     TRINIX_CASE(2)
@@ -801,6 +806,7 @@ hipError_t launch_feat(const FwdParams& p, int feat, hipStream_t st) {
     }
   }
 #undef TRINIX_CASE
+#undef TRINIX_KERNEL
   return hipErrorNotSupported;
 }
 
@@ -814,7 +820,7 @@ hipError_t launch_feat_plain(const FwdParams& p, int feat, hipStream_t st) {
 #define TRINIX_CASE(F)                                                                                          \
   case F:                                                                                                       \
     return launch_kernel(&attn_fwd_mfma16<E, D, BN, NW, OCC, KS, (F & kFeatAlibi) != 0, false, 0,             \
-                                          (F & kFeatQNorm) != 0>,                                              \
+                                          (F & kFeatQNorm) != 0, false>,                                       \
                          grid, block, 0, st, p);
     TRINIX_CASE(0)
     TRINIX_CASE((kFeatAlibi))
@@ -832,9 +838,10 @@ hipError_t launch_feat_plain(const FwdParams& p, int feat, hipStream_t st) {
 template <class E, int D>
 hipError_t launch_feat_split(const FwdParams& p, int feat, hipStream_t st) {
   const dim3 grid((unsigned)p.total_work), block(4 * 64);
-  if (feat == 0) return launch_kernel(&attn_fwd_mfma16<E, D, 64, 4, 2, 0, false, false, 0, false>, grid, block, 0, st, p);
+  if (feat == 0)
+    return launch_kernel(&attn_fwd_mfma16<E, D, 64, 4, 2, 0, false, false, 0, false, false>, grid, block, 0, st, p);
   if (feat == kFeatAlibi)
-    return launch_kernel(&attn_fwd_mfma16<E, D, 64, 4, 2, 0, true, false, 0, false>, grid, block, 0, st, p);
+    return launch_kernel(&attn_fwd_mfma16<E, D, 64, 4, 2, 0, true, false, 0, false, false>, grid, block, 0, st, p);
   return hipErrorNotSupported;
 }
 
