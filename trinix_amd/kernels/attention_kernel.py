@@ -381,7 +381,7 @@ def _launch_cached(key, q, k, v, rotary_cos, rotary_sin):
 # (and keep map) per call as on the full path.
 class _TrainLaunch:
     __slots__ = ("fwd", "bwd", "out_shape", "lse_shape", "dtype", "device", "align", "km_bytes", "do_stride",
-                 "dk_shape", "ws_bytes", "pad", "do_align")
+                 "dk_shape", "ws_bytes", "pieces", "pad", "do_align")
 
     def __init__(self, fwd, out_shape, lse_shape, dtype, device, align, km_bytes, dk_shape, pad, do_align):
         self.fwd = fwd                # AttnFwdArgs with null data pointers and seed
@@ -394,7 +394,8 @@ class _TrainLaunch:
         self.km_bytes = km_bytes      # dropout keep map bytes (0: none)
         self.do_stride = None         # dout strides the backward template was built for
         self.dk_shape = dk_shape      # shape of k (and of dk, dv)
-        self.ws_bytes = 0             # workspace of the backward
+        self.ws_bytes = 0             # workspace of the backward, planned under
+        self.pieces = None            # this TRINIX_BWD_PIECES
         self.pad = pad                # _Pad of q, k and v (a head_dim between the kernels'), or None
         self.do_align = do_align      # byte alignment dout needs
 
@@ -784,7 +785,7 @@ def _backward(state, dout):
         tpl.dropout_keep_map = None
         tpl.dropout_seed = 0
         ent.do_stride = tuple(do.stride())
-        ent.ws_bytes = wsb.value
+        ent.ws_bytes, ent.pieces = wsb.value, os.environ.get("TRINIX_BWD_PIECES")
         ent.bwd = tpl
     if d_out != D:
         dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
@@ -793,8 +794,9 @@ def _backward(state, dout):
 
 def _backward_cached(state, ent, dout):
     """(dq, dk, dv) through the layout's backward template, or None when
-    dout is not laid out as the template's."""
-    if dout.dtype != ent.dtype or dout.stride() != ent.do_stride or dout.data_ptr() % ent.do_align:
+    dout is not laid out as the template's or the plan's switch changed."""
+    if (dout.dtype != ent.dtype or dout.stride() != ent.do_stride or dout.data_ptr() % ent.do_align
+            or os.environ.get("TRINIX_BWD_PIECES") != ent.pieces):
         return None
     dev = ent.device
     a = nat.AttnBwdArgs.from_buffer_copy(ent.bwd)
