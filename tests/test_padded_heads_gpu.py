@@ -106,3 +106,20 @@ def test_padded_heads_output_written_before_the_backward(D):
         got = torch.autograd.grad(triton_attn_func(*leaves).mul_(0.5), leaves, ts[3] * 2)
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+def test_empty_operands_take_the_general_path():
+    """No head_dim columns: an empty output (and empty gradients) where the
+    caller gives the scale; no rows or keys: the forward's own error."""
+    q, k = torch.empty(2, 5, 3, 0, dtype=torch.bfloat16, device=DEV), torch.empty(2, 7, 3, 0, dtype=torch.bfloat16, device=DEV)
+    for _ in range(2):
+        assert triton_attn_func(q, k, k, softmax_scale=1.0).shape == (2, 5, 3, 0)
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, k)]
+        out = triton_attn_func(*leaves, softmax_scale=1.0)
+        grads = torch.autograd.grad(out, leaves, torch.empty_like(out))
+        assert [g.shape for g in grads] == [q.shape, k.shape, k.shape]
+    for Sq, Sk in ((0, 7), (5, 0)):
+        for D in (72, 100):
+            q, k = (torch.empty(2, n, 3, D, dtype=torch.bfloat16, device=DEV) for n in (Sq, Sk))
+            with pytest.raises(ValueError, match="trinix_attn_fwd.*: invalid or inconsistent sizes"):
+                triton_attn_func(q, k, k)

@@ -529,7 +529,7 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
         rotary_cos = rotary_sin = None
 
     pad = None
-    if d_kernel != D and q.dtype != torch.float32:
+    if d_kernel != D and q.dtype != torch.float32 and q.numel() and k.numel():
         # zero-padded in one launch; where the kernels can, they read and
         # write the other tensors at their own D columns ("narrow")
         ts = tuple(t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
