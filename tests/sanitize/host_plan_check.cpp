@@ -241,6 +241,43 @@ int main() {
             ++cases;
           }
   }
+  // ---- the forward's shape on small grids at head_dim 128 (figures beside
+  // key_split, host_plan.cpp): where the key split of 32-key tiles loses, the
+  // shape without it
+  {
+    struct Case {
+      int64_t B, Sq, Sk, Hq, Hkv;
+      int causal;
+      int64_t window;  // 0: none
+      int nw, bn, ks;
+    } table[] = {
+        {1, 1500, 1500, 8, 8, 0, 0, 4, 32, 2},       // 96 workgroups
+        {1, 200, 200, 30, 30, 0, 0, 4, 32, 2},       // 60, chain 4
+        {1, 130, 130, 30, 30, 0, 0, 4, 64, 1},       // 60, chain 3
+        {1, 1024, 1024, 24, 24, 0, 0, 4, 32, 2},     // 192 of full rows, chain 16
+        {1, 768, 768, 24, 24, 0, 0, 4, 64, 1},       // 144, chain 12
+        {1, 640, 640, 48, 48, 0, 0, 4, 64, 1},       // 240, chain 10
+        {1, 2048, 2048, 16, 16, 0, 0, 4, 64, 1},     // 256: full rows
+        {8, 128, 2048, 32, 32, 0, 0, 8, 128, 1},     // 256 pairs of 128 full rows: the wide shape
+        {1, 4096, 4096, 8, 8, 1, 512, 4, 64, 1},     // a window's even rows, 256
+        {1, 4096, 4096, 6, 6, 1, 1024, 4, 32, 2},    // the same, 192, chain 18
+        {1, 640, 640, 48, 48, 1, 0, 4, 32, 2},       // causal, head groups dealt evenly, chain 10
+        {1, 700, 700, 28, 28, 1, 0, 4, 64, 1},       // not evenly, chain 11
+        {1, 1024, 1024, 30, 30, 1, 0, 4, 64, 1},     // chain 16
+        {1, 1200, 1200, 20, 20, 1, 0, 4, 32, 2},     // chain 19
+        {1, 1024, 1024, 32, 4, 1, 0, 4, 64, 1},      // four groups of eight q-heads
+    };
+    for (const Case& c : table) {
+      trinix_attn_fwd_args a = valid_fwd();
+      a.batch = c.B, a.seqlen_q = c.Sq, a.seqlen_k = c.Sk, a.nheads_q = c.Hq, a.nheads_kv = c.Hkv, a.causal = c.causal;
+      a.has_window = c.window > 0, a.window_left = c.window;
+      FwdPlan pl;
+      CHECK(validate_fwd_args(&a) == TRINIX_OK && plan_fwd(&a, &pl) == TRINIX_OK, "key split case");
+      CHECK(pl.cfg.nw == c.nw && pl.cfg.bn == c.bn && pl.cfg.ks == c.ks, "key split case %d: (%d, %d, %d)", cases, pl.cfg.nw,
+            pl.cfg.bn, pl.cfg.ks);
+      ++cases;
+    }
+  }
   // ---- the tuning override TRINIX_ATTN_CFG="nw,occ,bn[,ks]": ks 0 (the
   // per-item split), 1 and 2 are taken, anything else leaves the planner's
   // choice

@@ -80,32 +80,47 @@ static bool wide_grid(int64_t batch, int64_t hq, int64_t sq, bool banded) {
 // whose wavefront pairs take alternate 32-key tiles, where 128-row workgroups
 // leave CUs idle or one wavefront per SIMD, and the longest row block's
 // `chain` of 64-key tiles is worth halving against the merge.  Head_dim 128
-// runs two workgroups per CU (64 KiB of LDS), so up to one 128-row workgroup
-// per CU; head_dim 256 runs one, so up to half of that.  Measured, bf16,
-// graph-timed kernel, us without | with the split:
-//   D=128 causal, workgroups x chain: 32 x 4 9.3 | 8.8, 96 x 11 16.7 | 15.3, 120 x 6
-//     12.5 | 11.9, 240 x 10 17.2 | 16.2, 256 x 16 23.8 | 21.7, 256 x 32 39.9 |
-//     35.3, 192 x 32 40.4 | 41.0; full rows 96 x 24 31.2 | 25.8, 240 x 24 35.6 |
-//     34.1; ALiBi 256 x 32 47.2 | 41.9; where it loses: 32 x 2 7.7 | 8.0, 128 x 3
-//     8.4 | 8.8, 256 x 8 16.6 | 17.2, 384 x 16 27.9 | 30.2, 512 x 32 49.9 | 52.0
-//   D=256 48 x 11 31.3 | 27.0, 128 x 32 76.7 | 60.0, full rows 128 x 16 44.6 |
-//     36.7; loses: 128 x 3 14.2 | 15.2, 192 x 8 27.8 | 31.8, 192 x 24 full 62.7 |
-//     85.5, 192 x 32 75.2 | 81.5
-static bool key_split(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, int64_t chain) {
-  if (head_dim < 128 || chain < 4 || batch * hq > kSmallGrid) return false;
-  const int64_t wgs = batch * hq * ((sq + 127) / 128);
-  return wgs <= kSmallGrid / 2 || (head_dim == 128 && wgs <= kSmallGrid && chain >= 10);
+// runs two workgroups per CU (64 KiB of LDS), head_dim 256 one.  Measured, bf16,
+// graph-timed kernel, speedup by the split (grids of bh x row blocks):
+//   up to 128 workgroups, D=128: full rows chain 6 1.10..1.13, 16 1.18, 48 1.24;
+//     causal chain 8 1.09, 10 1.13, 20 1.19; D=256 48 x 11 31.3 | 27.0 us, 128 x 32
+//     76.7 | 60.0; it loses at chain 2 and 3 (7.7 | 8.0, 8.4 | 8.8 us) and at D=256
+//     above (192 x 8 27.8 | 31.8, 192 x 32 75.2 | 81.5)
+//   129..256, D=128, full rows (and windows, whose rows are even too): up to 224
+//     workgroups chain 6..10 0.96..0.98, 12 0.99..1.00, 14 1.00..1.01, 20 1.02..1.05,
+//     48 1.03..1.12; 240 0.97..1.02 and 256 0.96..1.01 at any chain
+//   129..256, D=128, causal: with the head groups dealt evenly to the XCDs, and so
+//     dispatched longest rows first (fwd_item), chain 10 1.05, 16 1.09, 32 1.07;
+//     otherwise 10 0.96..1.02, 11 0.91..0.94, 12 0.96, 16 0.98..1.01, 18
+//     1.01..1.09, 32 1.07
+//   beyond: 384 x 16 27.9 | 30.2 us, 512 x 32 49.9 | 52.0
+static bool key_split(const trinix_attn_fwd_args* a) {
+  const int64_t D = a->head_dim, bh = a->batch * a->nheads_q;
+  if (D < 128 || bh > kSmallGrid) return false;
+  // keys the longest 128-row block sees, in 64-key tiles
+  int64_t keys = a->causal ? std::min(a->seqlen_q, a->seqlen_k) : a->seqlen_k;
+  if (a->has_window) {
+    const int64_t right = a->causal ? 0 : std::max<int64_t>(0, clamp_window(a->window_right));
+    keys = std::min(keys, std::max<int64_t>(0, clamp_window(a->window_left)) + right + 128);
+  }
+  const int64_t chain = (keys + 63) / 64, wgs = bh * ((a->seqlen_q + 127) / 128);
+  if (wgs <= kSmallGrid / 2) return chain >= 4;
+  if (D != 128 || wgs > kSmallGrid) return false;
+  if (a->causal && !a->has_window) return chain >= (a->batch * a->nheads_kv % kXcds == 0 ? 10 : 18);
+  return chain >= 14 && wgs <= kSmallGrid * 7 / 8;
 }
 Cfg16 pick_cfg16(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, bool banded, bool plain,
-                 bool split_ok, int64_t chain) {
+                 bool split_ok, bool split_keys) {
   Cfg16 c{4, head_dim == 256 ? 1 : 2, 64, 1};
   // batch * hq * row blocks, without overflow (each factor < 2^31 here)
   if (head_dim == 64 && batch * hq <= kSmallGrid && batch * hq * ((sq + 127) / 128) <= kSmallGrid) c.ks = 2;
   else if (head_dim == 64 && split_ok && batch * hq <= 2 * kSmallGrid &&
            batch * hq * ((sq + 127) / 128) <= 2 * kSmallGrid)
     c.ks = 0;
+  // the wide shape where it applies: 256 (batch, q-head) pairs of at most 128
+  // full rows, 2048 keys 48.3 us wide, 55.1 with the key split
   if (head_dim == 128 && plain && wide_grid(batch, hq, sq, banded)) c = Cfg16{8, 2, 128, 1};
-  if (plain && key_split(head_dim, batch, hq, sq, chain)) c = Cfg16{4, c.occ, 32, 2};
+  else if (split_keys) c = Cfg16{4, c.occ, 32, 2};
   if (const char* env = getenv("TRINIX_ATTN_CFG")) {
     int nw = 0, occ = 0, bn = 0, ks = 1;
     // ks 1 or 2: wavefronts per 32-row group; 0: the per-item split
@@ -295,14 +310,8 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   const bool f32 = a->dtype == TRINIX_F32;
   const bool plain = !a->mask && !(a->dropout_p > 0.f);
   const bool split_ok = plain && a->causal && !a->has_window && !a->q_norm_weight;
-  // keys the longest 128-row block sees, in 64-key tiles
-  int64_t keys = a->causal ? std::min(a->seqlen_q, a->seqlen_k) : a->seqlen_k;
-  if (a->has_window) {
-    const int64_t right = a->causal ? 0 : std::max<int64_t>(0, clamp_window(a->window_right));
-    keys = std::min(keys, std::max<int64_t>(0, clamp_window(a->window_left)) + right + 128);
-  }
   Cfg16 cfg = pick_cfg16(a->head_dim, a->batch, a->nheads_q, a->seqlen_q, a->causal || a->has_window, plain,
-                         split_ok, (keys + 63) / 64);
+                         split_ok, plain && key_split(a));
   if (a->q_norm_weight && a->head_dim == 64) cfg.ks = 1;  // where the fused q RMSNorm is built without the key split
   pl->n_items = 0;
   pl->num_mblk = 0;

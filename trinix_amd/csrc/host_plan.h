@@ -35,9 +35,9 @@ int check_narrow(int32_t dtype, int64_t head_dim, int64_t d_out);
 // Tile configuration of the 16-bit forward for a problem: `banded` when
 // causal or windowed, `plain` without a mask or dropout, `split_ok` when the
 // per-item key split applies (causal, no window, no mask, dropout or fused
-// q norm), `chain` 64-key tiles in the longest row block.
+// q norm), `split_keys` when the key split of head_dim 128 and 256 pays.
 Cfg16 pick_cfg16(int64_t head_dim, int64_t batch, int64_t hq, int64_t sq, bool banded, bool plain,
-                 bool split_ok = false, int64_t chain = 0);
+                 bool split_ok = false, bool split_keys = false);
 // Work items of the per-item key split for a causal problem of `heads`
 // (batch * q-heads) row sequences, row blocks of `rows` (= 32 * nw) rows and
 // `bn`-key tiles: the longest row blocks (tile count above half the longest)
