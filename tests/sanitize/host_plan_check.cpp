@@ -278,6 +278,28 @@ int main() {
       ++cases;
     }
   }
+  // ---- the decode launch's chunk count and loads (figures beside
+  // decode_run_plan, host_plan.cpp): short rows in several rounds run unsplit
+  // and through the caches
+  {
+    struct Case {
+      int64_t B, Sk;
+      int n_splits, streamed;
+    } table[] = {{16, 8192, 2, 1}, {48, 2048, 2, 1}, {12, 8192, 8, 1}, {24, 8192, 4, 1}, {16, 1000, 2, 1},
+                 {32, 300, 1, 1},  {48, 300, 1, 0},  {64, 300, 1, 0},  {96, 300, 1, 0},  {128, 300, 1, 0},
+                 {12, 1000, 2, 0}, {128, 1000, 1, 1}};
+    for (const Case& c : table) {  // 32 q-heads, 8 KV heads of D = 128: 8 B items, 32 B rows to merge
+      trinix_attn_fwd_args a = valid_fwd();
+      a.batch = c.B, a.seqlen_q = 1, a.seqlen_k = c.Sk, a.nheads_q = 32, a.nheads_kv = 8;
+      SplitPlan pl;
+      bool streamed = false;
+      CHECK(validate_fwd_args(&a) == TRINIX_OK && make_split_plan(&a, &pl), "decode case");
+      decode_run_plan(&a, &pl, &streamed);
+      CHECK(pl.n_splits == c.n_splits && streamed == (c.streamed != 0), "decode case %d: %d chunks, streamed %d", cases,
+            pl.n_splits, (int)streamed);
+      ++cases;
+    }
+  }
   // ---- the tuning override TRINIX_ATTN_CFG="nw,occ,bn[,ks]": ks 0 (the
   // per-item split), 1 and 2 are taken, anything else leaves the planner's
   // choice

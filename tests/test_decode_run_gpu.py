@@ -15,7 +15,8 @@ CASES = [
     (32, 1, 513, 8, 8, 128, dict()),                      # 256 items: unsplit, streamed
     (24, 1, 300, 8, 8, 128, dict()),                      # 192: unsplit, CUs idle
     (20, 1, 700, 16, 8, 128, dict(window_size=(0, 600))),  # 160 items, 3 chunks, a window's span
-    (48, 1, 400, 8, 8, 128, dict()),                      # 384 items, 2 chunks each
+    (48, 1, 400, 8, 8, 128, dict()),                      # 384 items, short rows: unsplit, through the caches
+    (48, 1, 1200, 8, 8, 128, dict()),                     # 384 items, 2 chunks each, streamed in three rounds
     (2, 3, 5000, 8, 1, 128, dict()),                      # 2 items, 24 rows: two row groups per KV head
     (64, 1, 257, 4, 4, 64, dict()),                       # head_dim 64, one workgroup per CU
     (12, 1, 1000, 16, 16, 64, dict()),                    # head_dim 64, the planned count

@@ -517,25 +517,35 @@ bool make_split_plan(const trinix_attn_fwd_args* a, SplitPlan* pl) {
 }
 
 // The plan bounds the chunks (and fixes the workspace) at four workgroups per
-// CU; a launch runs the count among one to four workgroups per CU that costs
-// least.  A decode step is bound by HBM, and one workgroup on every CU already
-// saturates it: more only add chunks to merge and spread the reads.  Cost: the
-// read at 5.5 TB/s, times how unevenly whole workgroups fall on the CUs (a
-// workgroup alone on its CU in a partial grid reads up to 1 / 0.82 of its
-// share), 6% for more than one per CU, and 3 us for the merge.  Head_dim 64
-// (half the bytes per load) follows no such rule: one workgroup per CU where
-// that fills them, the plan's count otherwise (B=12 S=3000 16 heads: 1152
-// workgroups 34.8 us, 768 37.5, 192 39.6).
-// Measured, bf16, 8 KV heads of D=128 unless noted, caches cold, graph-timed,
-// us as planned | run: B=16 S=8192 113.7 | 99.9 (256 workgroups, non-temporal),
-// B=4 S=8000 36.4 | 30.6, B=24 S=4000 84.6 | 78.2 (192), B=48 S=2000 ceil-planned
-// 1152 86.3 | 81.6 (768), B=64 S=2000 104.6 | 98.2 (512, unsplit), B=16 S=1000
-// 23.4 | 19.1, B=16 S=3000 16 heads of D=64 47.4 | 37.9.
+// CU; a launch runs the count among the planned one and one to four workgroups
+// per CU that costs least.  A decode step is bound by HBM, and one workgroup on
+// every CU already saturates it: more only add chunks to merge and spread the
+// reads.  Cost, in us: the read at 5.5 TB/s, times how unevenly whole workgroups
+// fall on the CUs (a workgroup alone on its CU in a partial grid reads up to
+// 1 / 0.82 of its share), 6% for more than one per CU and 8% off for
+// non-temporal loads; 2 for each round after the first; for the merge 5, its
+// rows and the partial sums.  Over 212 grids (3 to 128 sequences, 300 to 8192
+// keys, 8 KV heads of D=128, caches cold, graph-timed) the count it takes is
+// within 1% of the best one in the mean and 13% at worst, and on the 146 of them
+// that were timed with the planned count 10% faster than that, at worst 5%
+// slower (B=56 S=3000 136.5 | 130.1).  Head_dim 64 (half the bytes per load)
+// follows no such rule: one workgroup per CU where that fills them, the plan's
+// count otherwise (B=12 S=3000 16 heads: 1152 workgroups 34.8 us, 768 37.5, 192
+// 39.6).
+// Measured, bf16, 8 KV heads of D=128 unless noted, us as planned | run: B=16
+// S=8192 113.7 | 99.9 (256 workgroups, non-temporal), B=4 S=8000 36.4 | 30.6,
+// B=24 S=4000 84.6 | 78.2 (192), B=64 S=2000 104.6 | 98.2 (512, unsplit), B=16
+// S=1000 23.4 | 19.1, B=16 S=3000 16 heads of D=64 47.4 | 37.9; short rows, unsplit |
+// two chunks: B=48 S=300 21.1 | 25.4, S=500 27.8 | 28.9, S=1000 50.0 | 47.4; B=12
+// S=1000 two | eight chunks 17.1 | 20.0.
 // Non-temporal K/V loads pay where the workgroups fill the CUs evenly (B=16
 // S=8192 107.8 | 99.9 us, B=32 S=8000 193 | 189) and lose where CUs idle in the
 // last round (192 workgroups 78.2 | 88.3, 384 90.9 | 94.2, 128 9.8 | 10.1) and at
 // head_dim 64 (B=16 S=3000 16 heads 39.6 | 44.2); with several row groups the
-// K/V are read again, from L2.
+// K/V are read again, from L2.  In several rounds of short rows they lose too
+// (300 keys, 512, 768 and 1024 workgroups 23.1 | 23.5, 31.6 | 32.7, 39.8 | 42.7;
+// 500 keys 55.1 | 55.3, 1000 78.1 | 77.6), in one round they gain (128 items of 300
+// keys, two chunks 13.1 | 12.6, 256 13.7 | 13.3).
 void decode_run_plan(const trinix_attn_fwd_args* a, SplitPlan* pl, bool* streamed) {
   const int64_t items = a->batch * a->nheads_kv * pl->RG, span = (int64_t)pl->khi - pl->klo;
   auto rounds = [&](int64_t n) { return (items * n + kSmallGrid - 1) / kSmallGrid; };
@@ -544,27 +554,34 @@ void decode_run_plan(const trinix_attn_fwd_args* a, SplitPlan* pl, bool* streame
     *chunk = ((span + n - 1) / n + 63) / 64 * 64;
     return (span + *chunk - 1) / *chunk;
   };
-  if (pl->n_splits > 1 && !getenv("TRINIX_SPLITKV_CFG")) {
-    const double read_us = 4.0 * items * span * a->head_dim / 5.5e6;
-    double best = 1e30;
-    int64_t best_n = pl->n_splits;
+  auto non_temporal = [&](int64_t n) {
+    return a->head_dim == 128 && pl->RG == 1 && uneven(n) <= 1.07 && (rounds(n) == 1 || span >= 512);
+  };
+  auto cost = [&](int64_t n) {
+    const double read_us = 4.0 * items * span * a->head_dim / 5.5e6, rows = (double)(a->batch * a->nheads_kv) * pl->M;
+    const double share = rounds(n) > 1 ? 1.06 * uneven(n) : std::max(1.0, 0.82 * uneven(n));
+    return read_us * share * (non_temporal(n) ? 0.92 : 1.0) + 2.0 * (rounds(n) - 1) +
+           (n > 1 ? 5.0 + rows / 400 + rows * n / 3000 : 0.0);
+  };
+  // several row groups and long rows in more than one round run as planned (16
+  // sequences of 16 queries, S=8192 325 us in two chunks | 342 unsplit)
+  const bool as_planned = pl->RG > 1 && items > kSmallGrid && span > 3000;
+  if (pl->n_splits > 1 && !as_planned && !getenv("TRINIX_SPLITKV_CFG")) {
+    int64_t best_n = pl->n_splits, chunk;
     for (int k = 1; k <= 4; ++k) {
-      int64_t n = std::min<int64_t>(pl->n_splits, kSmallGrid * k / items), chunk;
+      int64_t n = std::min<int64_t>(pl->n_splits, kSmallGrid * k / items);
       if (n < 1) continue;
       n = run(n, &chunk);
-      if (a->head_dim == 64 && (k > 1 || uneven(n) > 1.07)) break;
-      const double share = rounds(n) > 1 ? 1.06 * uneven(n) : std::max(1.0, 0.82 * uneven(n));
-      const double us = read_us * share + (n > 1 ? 3.0 : 0.0);
-      if (us < best) {
-        best = us;
-        best_n = n;
+      if (a->head_dim == 64) {
+        if (k == 1 && uneven(n) <= 1.07) best_n = n;
+        break;
       }
+      if (cost(n) < cost(best_n)) best_n = n;
     }
-    int64_t chunk;
     pl->n_splits = (int)run(best_n, &chunk);
     pl->chunk = (int)chunk;
   }
-  *streamed = a->head_dim == 128 && pl->RG == 1 && uneven(pl->n_splits) <= 1.07;
+  *streamed = non_temporal(pl->n_splits);
 }
 
 }  // namespace trinix
