@@ -488,8 +488,11 @@ __global__ __launch_bounds__(NW * 64, (MASK && D == 64 && DROP != 2) ? 3 : OCC) 
   // is a wavefront's own chain (one per SIMD): MFMA 0.85 us of a 2.4 us tile, as
   // long again in LDS reads by the four wavefronts; operand reads 4, 6 or 8
   // ahead instead of 2 change nothing.
+  // ALiBi alone, unsplit, is the one variant that loses (bf16, us without |
+  // with, S=2048: 16 heads causal 94.4 | 97.1, 64 heads full rows 366 | 374; split, 8
+  // heads, 76.1 | 73.4; with a mask 220 | 214, with dropout 112 | 110).
   auto pin_acc = [&]() __attribute__((always_inline)) {
-    if constexpr (D == 256) {
+    if constexpr (D == 256 && (!ALIBI || MASK || DROP || KS == 2)) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) asm volatile("" : "+a"(acc[db]));
     }
