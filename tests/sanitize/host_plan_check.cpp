@@ -300,6 +300,40 @@ int main() {
       ++cases;
     }
   }
+  // ---- wavefronts per 32 rows or keys of the fp32 and head_dim 256 kernels
+  // (figures beside two_per_group, host_plan.cpp)
+  {
+    struct Case {
+      int dtype;
+      int64_t D, B, S, H;
+      int causal, fwd, dkdv, dq;
+    } table[] = {
+        {TRINIX_F32, 64, 4, 1024, 12, 1, 2, 2, 2},  {TRINIX_F32, 64, 8, 1024, 16, 1, 2, 2, 2},
+        {TRINIX_F32, 64, 16, 1024, 16, 1, 1, 1, 2}, {TRINIX_F32, 64, 128, 256, 16, 1, 1, 1, 1},
+        {TRINIX_F32, 64, 4, 1024, 12, 0, 2, 2, 2},  {TRINIX_F32, 64, 4, 1024, 16, 0, 1, 1, 1},
+        {TRINIX_F32, 64, 7, 1024, 16, 0, 2, 2, 2},  {TRINIX_F32, 64, 32, 1024, 16, 0, 1, 1, 1},
+        {TRINIX_F32, 128, 6, 1024, 8, 1, 2, 2, 2},  {TRINIX_F32, 128, 8, 1024, 8, 1, 1, 1, 2},
+        {TRINIX_F32, 128, 2, 1024, 8, 0, 2, 2, 2},  {TRINIX_F32, 128, 3, 1024, 8, 0, 1, 1, 1},
+        {TRINIX_F32, 128, 6, 1024, 8, 0, 2, 2, 2},  {TRINIX_F32, 256, 1, 1024, 8, 1, 1, 1, 1},
+        {TRINIX_BF16, 256, 2, 1024, 8, 1, 1, 2, 2}, {TRINIX_BF16, 256, 2, 2048, 8, 1, 1, 1, 2},
+        {TRINIX_BF16, 256, 2, 1024, 8, 0, 1, 1, 2}, {TRINIX_F16, 256, 2, 1024, 8, 0, 1, 1, 1},
+        {TRINIX_F16, 256, 2, 1024, 8, 1, 1, 2, 2},  {TRINIX_F16, 256, 2, 2048, 8, 1, 1, 1, 1},
+    };
+    for (const Case& c : table) {
+      trinix_attn_fwd_args f = valid_fwd();
+      trinix_attn_bwd_args b = valid_bwd();
+      f.batch = b.batch = c.B, f.seqlen_q = f.seqlen_k = b.seqlen_q = b.seqlen_k = c.S;
+      f.nheads_q = f.nheads_kv = b.nheads_q = b.nheads_kv = c.H, f.head_dim = b.head_dim = c.D;
+      f.dtype = b.dtype = c.dtype, f.causal = b.causal = c.causal;
+      FwdPlan fp;
+      BwdPlan bp;
+      CHECK(validate_fwd_args(&f) == TRINIX_OK && validate_bwd_args(&b) == TRINIX_OK && plan_fwd(&f, &fp) == TRINIX_OK &&
+                plan_bwd(&b, &bp) == TRINIX_OK, "wavefronts per group case");
+      CHECK(fp.f32_ks == c.fwd && bp.kv_ks == c.dkdv && bp.dq_ks == c.dq, "wavefronts per group case %d: %d, %d, %d", cases,
+            fp.f32_ks, bp.kv_ks, bp.dq_ks);
+      ++cases;
+    }
+  }
   // ---- the tuning override TRINIX_ATTN_CFG="nw,occ,bn[,ks]": ks 0 (the
   // per-item split), 1 and 2 are taken, anything else leaves the planner's
   // choice

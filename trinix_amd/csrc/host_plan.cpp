@@ -292,19 +292,34 @@ int64_t clamp_window(int64_t w) {
 
 // Two wavefronts per 32 keys or rows (half the chain of tiles, twice the
 // workgroups, but twice the tile copies per product and a merge through LDS)
-// in the fp32 and head_dim 256 kernels, where `wgs` workgroups of one
-// wavefront per 32 would leave the chip with few rounds.  Measured (forward +
-// backward, us, one | two wavefronts):
-//   dK/dV  fp32 D=64 384 workgroups 402 | 344, 1024: 1435 | 1410; D=128 288:
-//          430 | 379, 512: 1448 | 1468; D=256 bf16 256: 432 | 344, 4096: 4030 |
-//          4430, fp16 256: 502 | 400, 512: 395 | 421
-//   dQ     fp32 D=64 384: 408 | 344, 1024: 1519 | 1410; D=128 288: 398 | 379,
-//          512: 1670 | 1468; D=256 bf16 256: 367 | 344, 2048: 4030 | 4300, fp16
-//          512: 395 | 423
-//   forward (fp32) D=64 384: 111 | 79, 1024: 325 | 313; D=128 512: 331 | 353
-static bool two_per_group(int64_t head_dim, int64_t wgs, int64_t limit128) {
-  return wgs <= (head_dim == 64 ? 4096 : head_dim == 128 ? limit128 : 384);
+// in the fp32 and head_dim 256 kernels; `wgs` workgroups of one wavefront per 32.
+// Rows of even length: where halves of a workgroup, each 4..10% dearer, take
+// fewer rounds of the CUs.  Measured, us, one | two (fp32 S=1024, the backward's
+// other kernel at its best):
+//   D=64 forward 96 workgroups 96 | 59, 384 158 | 132, 512 161 | 165, 768 230 | 237, 896
+//     300 | 277, 1024 301 | 316; dK/dV + dQ 384 480 | 398, 512 488 | 505, 896 937 | 866,
+//     4096 3678 | 3868
+//   D=128 forward 128 162 | 97, 192 164 | 178, 384 317 | 268, 512 323 | 350; backward 192
+//     495 | 526, 384 967 | 793, 512 983 | 1046
+//   D=256 bf16 dK/dV (two workgroups a block) 128 147 | 125, 256 160 | 175, 384 228 | 220,
+//     512 419 | 469; dQ 64 147 | 130, 128 160 | 143, 192 228 | 246
+// Causal rows, whose blocks differ in length, longest first: up to `limit`.
+//   D=64 forward 512 128 | 109, 896 170 | 163, 1024 184 | 182, 1536 259 | 260, 2048 333 |
+//     343, 4096 647 | 682; dK/dV 512 424 | 389, 1024 728 | 717, 1536 987 | 1007, 4096 2464 |
+//     2528; dQ 1024 728 | 634, 4096 2464 | 2319, 5120 3055 | 2859 (half the
+//     diagonal's waste: at any count)
+//   D=128 forward 256 163 | 107, 384 166 | 165, 512 192 | 201; dK/dV 384 597 | 592, 512 738 |
+//     754; dQ 384 597 | 549, 1024 1374 | 1293, 1280 1666 | 1617
+//   D=256 bf16 dK/dV 256 381 | 300, 512 285 | 316; dQ 256 285 | 266, 512 445 | 478; fp16 dQ
+//     (two workgroups a block) 256 157 | 150, 512 325 | 350
+//   and of at most 256 rows as even ones: dQ D=64 S=256 4096 894 | 944, D=128 512 266 | 285
+static bool two_per_group(int64_t head_dim, bool even, int64_t wgs, int64_t limit) {
+  if (!even) return wgs <= limit;
+  const double dearer = head_dim == 64 ? 1.04 : head_dim == 128 ? 1.08 : 1.1;
+  return dearer * (double)((2 * wgs + kSmallGrid - 1) / kSmallGrid) < 2.0 * (double)((wgs + kSmallGrid - 1) / kSmallGrid);
 }
+// Whether the blocks of a problem are of (nearly) one length.
+static bool even_rows(int32_t causal, int32_t has_window, int64_t sq) { return !causal || has_window || sq <= 256; }
 
 int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   const bool f32 = a->dtype == TRINIX_F32;
@@ -317,7 +332,9 @@ int plan_fwd(const trinix_attn_fwd_args* a, FwdPlan* pl) {
   pl->num_mblk = 0;
   pl->f32_ks = 1;
   if (f32 && a->head_dim <= 128) {
-    pl->f32_ks = two_per_group(a->head_dim, a->batch * a->nheads_q * ((a->seqlen_q + 127) / 128), 384) ? 2 : 1;
+    pl->f32_ks = two_per_group(a->head_dim, even_rows(a->causal, a->has_window, a->seqlen_q),
+                               a->batch * a->nheads_q * ((a->seqlen_q + 127) / 128), a->head_dim == 64 ? 1024 : 384)
+                     ? 2 : 1;
     if (const char* env = getenv("TRINIX_F32_KS"))  // tuning and tests
       if (env[0] == '1' || env[0] == '2') pl->f32_ks = env[0] - '0';
   }
@@ -424,8 +441,11 @@ int plan_bwd(const trinix_attn_bwd_args* a, BwdPlan* pl, bool split) {
       pl->dq_hs = a->dtype == TRINIX_BF16 ? 1 : 2;
     }
     if (!(f32 && D == 256)) {  // (whose tiles fill the LDS)
-      pl->kv_ks = two_per_group(D, a->batch * a->nheads_kv * ((a->seqlen_k + 127) / 128) * pl->kv_hs, 384) ? 2 : 1;
-      pl->dq_ks = two_per_group(D, a->batch * a->nheads_q * ((a->seqlen_q + 127) / 128) * pl->dq_hs, 1024) ? 2 : 1;
+      const bool even = even_rows(a->causal, a->has_window, a->seqlen_q);
+      const int64_t kv = a->batch * a->nheads_kv * ((a->seqlen_k + 127) / 128) * pl->kv_hs;
+      const int64_t dq = a->batch * a->nheads_q * ((a->seqlen_q + 127) / 128) * pl->dq_hs;
+      pl->kv_ks = two_per_group(D, even, kv, D == 64 ? 1024 : 384) ? 2 : 1;
+      pl->dq_ks = two_per_group(D, even, dq, D == 256 ? 384 : 1ll << 31) ? 2 : 1;
       if (const char* env = getenv("TRINIX_BWD_GENERIC")) {  // "dq_ks,kv_ks" (tuning and tests)
         int ks = 0, kks = 0;
         if (sscanf(env, "%d,%d", &ks, &kks) == 2 && (ks == 1 || ks == 2) && (kks == 1 || kks == 2)) {
