@@ -1,6 +1,7 @@
-"""GPU tests of the kernels whose P and dZ keep fp32 precision in their
-products: the fp32 forward and backward, and the 16-bit backward at head_dim
-256 (``csrc/attn_fwd_f32.hip``, ``csrc/attn_bwd_generic.h``), at the edges of
+"""GPU tests of the kernels whose P and dZ enter their products with more bits
+than a 16-bit operand has: the fp32 forward and backward (24 bits), and the
+16-bit backward at head_dim 256 (two 16-bit terms: 16 bits in bf16, about 21 in
+fp16) (``csrc/attn_fwd_f32.hip``, ``csrc/attn_bwd_generic.h``), at the edges of
 their 32-row tiles and 64/128-row blocks, with one and with two wavefronts per
 32 keys or rows.
 

@@ -3,8 +3,8 @@
 // trinix_attn_bwd validates the arguments, computes delta = rowsum(dO * O)
 // into the caller's workspace and launches the dK/dV and dQ kernels: the
 // bf16/fp16 MFMA pipeline (attn_bwd16.h, instantiated per (dtype, head_dim)
-// in attn_bwd16_*.hip) for head_dim 64/128, the kernels whose P and dZ keep
-// fp32 precision (attn_bwd_generic.h, attn_bwd_generic_*.hip) for fp32 and head_dim 256.
+// in attn_bwd16*.hip) for head_dim 64/128, the kernels of attn_bwd_generic.h
+// (attn_bwd_generic_*.hip) for fp32 and head_dim 256.
 #include <cstdint>
 
 #include "attn_bwd_generic.h"

@@ -7,25 +7,10 @@
 #include <atomic>
 #include <cstring>
 
-#include <cstdio>
-#include <cstdlib>
-
 #include "attn_params.h"
 #include "host_plan.h"
 
-namespace trinix {
-
-}  // namespace trinix
-
-// ---------------------------------------------------------------------------
-// Host side: validation, tile table, launch.
-// ---------------------------------------------------------------------------
 using namespace trinix;
-
-namespace {
-
-
-}  // namespace
 
 extern "C" {
 

@@ -1,7 +1,7 @@
-// Operand policies of the attention kernels that keep every coefficient
-// (P, dZ) at fp32 precision in its products: what a tile of 32 rows looks
-// like in LDS, how a wavefront forms a 32x32 block of row products from it,
-// and how it adds tile^T * coefficients to its accumulators.
+// Operand policies of the attention kernels whose coefficients (P, dZ) enter
+// their products with more bits than a 16-bit operand has: what a tile of 32
+// rows looks like in LDS, how a wavefront forms a 32x32 block of row products
+// from it, and how it adds tile^T * coefficients to its accumulators.
 //
 // Common shape: a wavefront owns 32 columns (keys in dK/dV, query rows in dQ
 // and the forward); lane l holds column l % 32, whose own rows (K and V, or Q
@@ -16,8 +16,9 @@
 //                        blocks from db0 (a multiple of NDB).
 //
 //   Ops32  fp32 operands on v_mfma_f32_32x32x2f32 (exact products, fp32 sums);
-//          an operand element is 4 bytes, so neither product needs a
-//          transposed copy and P / dZ never leave the registers.
+//          the coefficients keep all 24 bits; an operand element is 4 bytes,
+//          so neither product needs a transposed copy and P / dZ never leave
+//          the registers.
 //   Ops16  16-bit operands on v_mfma_f32_32x32x16; the coefficients enter as
 //          two 16-bit terms x = hi + lo, hi = round(x), lo = round(x - hi): 16
 //          (bf16) or 21 (fp16) significant bits, two MFMAs per operand read.

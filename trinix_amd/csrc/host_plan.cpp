@@ -32,7 +32,8 @@ int check_tensor(const void* ptr, const int64_t st[4], int esize) {
   return TRINIX_OK;
 }
 
-// fp32 BSHD tensor (generic kernels, element loads): head_dim stride 1.
+// fp32 BSHD tensor: head_dim stride 1, 4-byte aligned, any other stride (the
+// kernels copy rows 16 bytes a lane where rows_aligned16 allows, else 4).
 int check32(const void* ptr, const int64_t st[4]) {
   if (!ptr) return TRINIX_ERR_NULL_POINTER;
   if (st[3] != 1 || ((uintptr_t)ptr & 3) != 0) return TRINIX_ERR_BAD_STRIDE;
