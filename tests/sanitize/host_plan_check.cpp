@@ -140,7 +140,7 @@ static void check_bwd_grids(const trinix_attn_bwd_args& a, int rc, const BwdPlan
   CHECK((wide)pl.ws_bytes == (pl.kv_T ? bkv * pl.kv_P * 2 * 128 * a.head_dim * 4 : 0), "piece workspace");
 }
 
-int main() {
+int main(int argc, char** argv) {
   int cases = 0;
   // ---- status codes of the forward's validation
   {
@@ -445,10 +445,39 @@ int main() {
   // a share of the fuzz's accepted argument sets (sampled items)
   bounds::Report BR;
   int modelled = 0;
+  long pieced = 0, generic = 0, narrow = 0;
+  auto bwd_of = [](const trinix_attn_fwd_args& f) {
+    trinix_attn_bwd_args b = valid_bwd();
+    b.batch = f.batch, b.seqlen_q = f.seqlen_q, b.seqlen_k = f.seqlen_k, b.nheads_q = f.nheads_q;
+    b.nheads_kv = f.nheads_kv, b.head_dim = f.head_dim, b.dtype = f.dtype, b.causal = f.causal;
+    b.has_window = f.has_window, b.window_left = f.window_left, b.window_right = f.window_right;
+    b.mask = f.mask, b.mask_dtype = f.mask_dtype, b.mask_blockmap = f.mask_blockmap, b.dropout_p = f.dropout_p;
+    b.dropout_keep_map = f.dropout_keep_map;
+    for (int i = 0; i < 4; ++i) {
+      b.q_stride[i] = b.dout_stride[i] = b.out_stride[i] = b.dq_stride[i] = f.q_stride[i];
+      b.k_stride[i] = b.dk_stride[i] = f.k_stride[i];
+      b.v_stride[i] = b.dv_stride[i] = f.v_stride[i];
+      b.mask_stride[i] = f.mask_stride[i];
+    }
+    return b;
+  };
+  auto model_pieces = [&](const trinix_attn_bwd_args& b) {
+    BwdPlan bp;
+    if (validate_bwd_args(&b) != TRINIX_OK || plan_bwd(&b, &bp, true) != TRINIX_OK || !bp.kv_T) return;
+    bounds::model_pieces(BR, b, bp);
+    ++pieced;
+  };
+  // `first`: the caller wants to know whether any check fails, not how many
+  const bool first = argc > 1 && std::strcmp(argv[1], "first") == 0;
   auto model_one = [&](const trinix_attn_fwd_args& f, int64_t limit) {
-    if (validate_fwd_args(&f) != TRINIX_OK || f.dtype == TRINIX_F32) return;
+    if (validate_fwd_args(&f) != TRINIX_OK || (first && BR.failures)) return;
     FwdPlan fp;
-    if (plan_fwd(&f, &fp) == TRINIX_OK) bounds::model_fwd16(BR, f, fp, limit);
+    const bool planned_fwd = plan_fwd(&f, &fp) == TRINIX_OK;
+    if (f.dtype == TRINIX_F32) {
+      if (planned_fwd) bounds::model_fwd_f32(BR, f, fp, limit);
+    } else if (planned_fwd) {
+      bounds::model_fwd16(BR, f, fp, limit);
+    }
     SplitPlan sp;
     if (make_split_plan(&f, &sp)) {
       bounds::model_decode(BR, f, sp, limit);
@@ -458,21 +487,19 @@ int main() {
       sp.ws_bytes = sp.n_splits > 1 ? slot * sp.n_splits : 0;
       bounds::model_decode(BR, f, sp, limit);
     }
-    if (f.head_dim <= 128 && f.q_norm_weight == nullptr) {
-      trinix_attn_bwd_args b = valid_bwd();
-      b.batch = f.batch, b.seqlen_q = f.seqlen_q, b.seqlen_k = f.seqlen_k, b.nheads_q = f.nheads_q;
-      b.nheads_kv = f.nheads_kv, b.head_dim = f.head_dim, b.dtype = f.dtype, b.causal = f.causal;
-      b.has_window = f.has_window, b.window_left = f.window_left, b.window_right = f.window_right;
-      b.mask = f.mask, b.mask_dtype = f.mask_dtype, b.mask_blockmap = f.mask_blockmap, b.dropout_p = f.dropout_p;
-      b.dropout_keep_map = f.dropout_keep_map;
-      for (int i = 0; i < 4; ++i) {
-        b.q_stride[i] = b.dout_stride[i] = b.out_stride[i] = b.dq_stride[i] = f.q_stride[i];
-        b.k_stride[i] = b.dk_stride[i] = f.k_stride[i];
-        b.v_stride[i] = b.dv_stride[i] = f.v_stride[i];
-        b.mask_stride[i] = f.mask_stride[i];
-      }
+    if (f.q_norm_weight == nullptr) {
+      const trinix_attn_bwd_args b = bwd_of(f);
       BwdPlan bp;
-      if (validate_bwd_args(&b) == TRINIX_OK && plan_bwd(&b, &bp) == TRINIX_OK) bounds::model_bwd16(BR, b, bp, limit);
+      if (validate_bwd_args(&b) == TRINIX_OK) {
+        if (plan_bwd(&b, &bp) == TRINIX_OK) {
+          if (bp.generic) bounds::model_bwd_generic(BR, b, bp, limit), ++generic;
+          else bounds::model_bwd16(BR, b, bp, limit);
+        }
+        model_pieces(b);
+        if (b.dtype != TRINIX_F32 && b.head_dim <= 128)
+          for (int64_t d : {(int64_t)8, b.head_dim / 2 + 8, b.head_dim - 8})
+            if (b.batch * b.nheads_q < (1ll << 31)) bounds::model_narrow(BR, b, d), ++narrow;
+      }
     }
     ++modelled;
   };
@@ -521,7 +548,46 @@ int main() {
     a = shape(1, 64, 64, 8, 8, 128, TRINIX_BF16), a.has_window = 1;                       // extreme windows
     a.window_left = std::numeric_limits<int64_t>::min(), a.window_right = std::numeric_limits<int64_t>::max(), add(a);
     a.window_left = std::numeric_limits<int64_t>::max(), a.window_right = std::numeric_limits<int64_t>::min(), add(a);
+    const int64_t inf = std::numeric_limits<int64_t>::max();
+    for (int64_t D : {64, 128, 256})  // fp32: 16-byte and odd row strides, every split
+      for (int64_t Sq : {1, 33, 128, 300})
+        for (int64_t Sk : {1, 64, 257})
+          for (int c = 0; c < 4; ++c) {
+            a = shape(2, Sq, Sk, 4, c % 2 ? 1 : 2, D, TRINIX_F32);
+            a.causal = c & 1;
+            if (c >= 2) a.has_window = 1, a.window_left = 40, a.window_right = c == 3 ? inf : -5;
+            if (c == 2) a.k_stride[1] += 1, a.q_stride[1] += 3;
+            if (c == 3) a.mask = (void*)4096, a.mask_dtype = TRINIX_F32, a.mask_blockmap = (const uint8_t*)4096,
+                        a.mask_stride[2] = Sk, a.mask_stride[3] = 1;
+            add(a);
+          }
+    a = shape(4, 1024, 1024, 12, 12, 64, TRINIX_F32), a.causal = 1, add(a);
+    a = shape(64, 1024, 1024, 16, 16, 64, TRINIX_F32), a.causal = 1, add(a);             // one wavefront per 32 rows
+    a = shape(2, 700, 700, 4, 4, 128, TRINIX_F32), a.k_stride[1] = a.v_stride[1] = (1ll << 24) - 4, add(a);
+    a.k_stride[1] = 1ll << 40, add(a);
+    a = shape(2, 2048, 2048, 8, 4, 256, TRINIX_BF16), a.causal = 1, add(a);
+    a = shape(16, 300, 300, 8, 8, 256, TRINIX_F16), a.k_stride[1] = (1ll << 22) - 8, add(a);
+    a = shape(2, 2048, 2048, 16, 4, 128, TRINIX_BF16), a.causal = 1, add(a);             // dK/dV in pieces
+    a = shape(1, 8192, 8192, 16, 4, 128, TRINIX_BF16), a.causal = 1, add(a);
+    a = shape(2, 1000, 1000, 16, 4, 64, TRINIX_F16), add(a);
     for (const auto& f : cur) model_one(f, kAll);
+    for (const char* both : {"1,1", "1,2", "2,1", "2,2"}) {  // every built split, whatever the plan takes
+      setenv("TRINIX_BWD_GENERIC", both, 1);
+      setenv("TRINIX_F32_KS", both, 1);
+      for (size_t k = 0; k < cur.size(); k += 3)
+        if (cur[k].dtype == TRINIX_F32 || cur[k].head_dim == 256) model_one(cur[k], kAll);
+      unsetenv("TRINIX_F32_KS");
+      unsetenv("TRINIX_BWD_GENERIC");
+    }
+    for (const char* pieces : {"1", "3", "20"}) {
+      setenv("TRINIX_BWD_PIECES", pieces, 1);
+      for (size_t k = 0; k < cur.size(); k += 2)
+        if (cur[k].seqlen_q <= 2048) model_pieces(bwd_of(cur[k]));
+      unsetenv("TRINIX_BWD_PIECES");
+    }
+    const int64_t pads[][5] = {{1, 1, 1, 1, 64}, {2, 70, 4, 36, 64}, {3, 17, 5, 80, 128}, {1, 9, 2, 63, 64}, {2, 5, 3, 160, 256}};
+    for (const auto& z : pads) bounds::model_pad(BR, z[0], z[1], z[2], z[3], z[4], true);
+    bounds::model_pad(BR, 1 << 19, 1 << 19, 64, 100, 128, false);
     cases += (int)cur.size();
   }
   {
@@ -538,6 +604,7 @@ int main() {
       a.nheads_q = a.nheads_kv * (int64_t)(1 + next_u64() % 8);
       a.head_dim = (int64_t)(64 << (next_u64() % 3));
       a.dtype = next_u64() % 2 ? TRINIX_BF16 : TRINIX_F16;
+      if (next_u64() % 4 == 0) a.dtype = TRINIX_F32;
       a.causal = (int32_t)(next_u64() % 2);
       a.has_window = (int32_t)(next_u64() % 2);
       a.window_left = rand_size();
@@ -554,7 +621,7 @@ int main() {
       }
       if (next_u64() % 4 == 0) {
         a.dropout_p = 0.1f;
-        if (a.head_dim <= 128) a.dropout_keep_map = (void*)4096;
+        if (a.head_dim <= 128 && a.dtype != TRINIX_F32) a.dropout_keep_map = (void*)4096;
       }
       if (validate_fwd_args(&a) != TRINIX_OK) continue;
       model_one(a, 4096);
@@ -562,6 +629,7 @@ int main() {
     }
     cases += ran;
   }
+  CHECK(pieced > 300 && generic > 500 && narrow > 1000, "modelled %ld plans in pieces, %ld generic, %ld narrow", pieced, generic, narrow);
   std::printf("bounds model: %d argument sets, %ld checks, %ld failures\n", modelled, BR.checks, BR.failures);
   failures += (int)BR.failures;
   std::printf("cases %d, fuzz accepted %d, planned %d, failures %d\n", cases, accepted, planned, failures);

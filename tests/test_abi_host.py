@@ -378,3 +378,57 @@ def test_splitkv_plan_invariants_random(lib):
         assert items * ns < 2 ** 31
         assert wb == (0 if ns == 1 else kw["batch"] * Hkv * rows * ns * (kw["head_dim"] + 1) * 4)
         assert wb <= nat.SPLITKV_SCRATCH_BYTES
+
+
+def test_narrow_and_padding_entry_points_reject_before_launch(lib):
+    """``trinix_attn_fwd_narrow``, ``trinix_attn_bwd_narrow`` and its workspace,
+    ``trinix_attn_bwd_ws`` and ``trinix_pad_heads``: the checks of the plain entry
+    points, then their own."""
+    def fwd(d_out, **kw):
+        return lib.trinix_attn_fwd_narrow(ctypes.byref(_args(**kw)), d_out, None)
+
+    def bwd(d_out, ws=4096, size=1 << 40, **kw):
+        return lib.trinix_attn_bwd_narrow(ctypes.byref(_bwd_args(**kw)), d_out, ws, size, None)
+
+    def space(d_out, **kw):
+        n = ctypes.c_int64(-1)
+        return lib.trinix_attn_bwd_narrow_workspace(ctypes.byref(_bwd_args(**kw)), d_out, ctypes.byref(n)), n.value
+
+    d256 = nat.int64x4((8 * 64 * 256, 8 * 256, 256, 1))
+    wide = {n + "_stride": d256 for n in ("q", "k", "v", "out")}
+    wide_bwd = {n + "_stride": d256 for n in ("q", "k", "v", "out", "dout", "dq", "dk", "dv")}
+    for call in (fwd, bwd, lambda d, **kw: space(d, **kw)[0]):
+        for d in (0, -8, 12, 63, 136, 1 << 40):  # not a multiple of 8 in (0, head_dim]
+            assert call(d) == nat.TRINIX_ERR_BAD_HEAD_DIM, d
+        assert call(80, dtype=nat.TRINIX_F32) == nat.TRINIX_ERR_BAD_HEAD_DIM
+        assert call(80, head_dim=256, **(wide if call is fwd else wide_bwd)) == nat.TRINIX_ERR_BAD_HEAD_DIM
+        assert call(80, seqlen_k=0) == nat.TRINIX_ERR_BAD_SHAPE
+        assert call(80, q=None) == nat.TRINIX_ERR_NULL_POINTER
+        assert call(80, head_dim=96) == nat.TRINIX_ERR_BAD_HEAD_DIM
+    # fused RoPE and q norm run over head_dim columns
+    assert fwd(80, rope_cos=4096, rope_sin=4096, rope_stride=64) == nat.TRINIX_ERR_BAD_ARGUMENT
+    assert fwd(80, q_norm_weight=4096, q_norm_eps=1e-6) == nat.TRINIX_ERR_BAD_ARGUMENT
+    # the padded dout (and the partial sums behind it, here none): 16-byte aligned and large enough
+    rc, n = space(80)
+    assert rc == 0 and n == 64 * 8 * 128 * 2 and space(128) == (0, 0)
+    for ws, size in ((None, n), (4096, n - 1), (4100, n)):
+        assert bwd(80, ws, size) == nat.TRINIX_ERR_BAD_ARGUMENT
+    assert lib.trinix_attn_bwd_narrow_workspace(ctypes.byref(_bwd_args()), 80, None) == nat.TRINIX_ERR_NULL_POINTER
+    assert lib.trinix_attn_fwd_narrow(None, 80, None) == nat.TRINIX_ERR_NULL_POINTER
+    assert lib.trinix_attn_bwd_narrow(None, 80, None, 0, None) == nat.TRINIX_ERR_NULL_POINTER
+    assert lib.trinix_attn_bwd_ws(None, None, 0, None) == nat.TRINIX_ERR_NULL_POINTER
+    assert lib.trinix_attn_bwd_ws(ctypes.byref(_bwd_args(batch=0)), None, 0, None) == nat.TRINIX_ERR_BAD_SHAPE
+
+    def pad(n=1, x=4096, out=8192, stride=(64, 8, 8, 1), sizes=(1, 8, 1), d=80, D=128, dtype=nat.TRINIX_BF16):
+        return lib.trinix_pad_heads(n, (ctypes.c_void_p * 3)(x, x, x), (ctypes.c_int64 * 12)(*(stride * 3)),
+                                    (ctypes.c_void_p * 3)(out, out, out), (ctypes.c_int64 * 9)(*(sizes * 3)), d, D, dtype,
+                                    None)
+
+    assert pad(dtype=nat.TRINIX_F32) == nat.TRINIX_ERR_BAD_DTYPE
+    assert pad(n=0) == pad(n=4) == nat.TRINIX_ERR_BAD_ARGUMENT
+    for d, D in ((0, 128), (-1, 128), (80, 72), (80, 84), (80, 1032)):
+        assert pad(d=d, D=D) == nat.TRINIX_ERR_BAD_HEAD_DIM, (d, D)
+    assert pad(x=None) == pad(out=None) == nat.TRINIX_ERR_NULL_POINTER
+    assert pad(sizes=(0, 8, 1)) == pad(sizes=(1, 1 << 30, 1)) == pad(sizes=(1, 8, -1)) == nat.TRINIX_ERR_BAD_SHAPE
+    assert pad(stride=(64, 8, 8, 2)) == pad(x=4097) == pad(out=8200) == nat.TRINIX_ERR_BAD_STRIDE
+    assert lib.trinix_pad_heads(1, None, None, None, None, 80, 128, nat.TRINIX_BF16, None) == nat.TRINIX_ERR_NULL_POINTER

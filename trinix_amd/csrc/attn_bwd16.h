@@ -260,7 +260,7 @@ __device__ inline int lane_piece_ends(const BwdParams& p, const Band& band, int 
 }
 __device__ inline int piece_block(const BwdParams& p, const Band& band, int lane, int index, int& np, int& pk) {
   const int end = lane_piece_ends(p, band, lane);
-  const int kblk = min((int)__popcll(__builtin_amdgcn_ballot_w64(end <= index)), p.num_kblk - 1);
+  const int kblk = bwd_piece_kblk((int)__popcll(__builtin_amdgcn_ballot_w64(end <= index)), p.num_kblk);
   const int hi = __builtin_amdgcn_readlane(end, kblk), lo = kblk ? __builtin_amdgcn_readlane(end, kblk - 1) : 0;
   np = hi - lo;
   pk = index - lo;
@@ -279,11 +279,11 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce(const BwdParams p) {
   const int end = lane_piece_ends(p, band, lane);
   const int hi = __builtin_amdgcn_readlane(end, kblk), lo = kblk ? __builtin_amdgcn_readlane(end, kblk - 1) : 0;
   if (hi - lo < 2) return;  // written by its only piece
-  const int unit = sl * 256 + tid, kg = unit / (DB * 4 * 64), dq = unit / 64 % (DB * 4), l = unit & 63;
-  const float* part = p.part + (((int64_t)group * p.kv_P + lo) * 2 + sb) * BK * D + unit * 4;
+  const int unit = sl * 256 + tid;
+  const float* part = p.part + bwd_part_base((int64_t)group * p.kv_P + lo, sb, D) + unit * 4;
   f32x4_t s = *(const f32x4_t*)part;
   for (int k = 1; k < hi - lo; ++k) s += *(const f32x4_t*)(part + (int64_t)k * 2 * BK * D);
-  const int j = kblk * BK + kg * 32 + (l & 31), d0 = dq * 8 + (l >> 5) * 4;
+  const int j = kblk * BK + bwd_part_key(unit, D), d0 = bwd_part_col(unit, D);
   if (j >= p.Sk || d0 >= p.d_out) return;
   const int b = group / p.Hkv, hkv = group % p.Hkv;
   uint16_t* row = sb ? p.dk + b * p.dk_sb + hkv * p.dk_sh + (int64_t)j * p.dk_ss
@@ -696,7 +696,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv(const BwdParams p) {
     // ---- epilogue: a piece's fp32 partial sums, in the order of the lanes
     // (bwd_dkdv_reduce adds them up)
     if (EXT && np > 1) {
-      float* part = p.part + ((int64_t)slot * 2 + (SB ? 1 : 0)) * BK * D + (kg * DB * 4 * 64 + lane) * 4;
+      float* part = p.part + bwd_part_base(slot, SB ? 1 : 0, D) + bwd_part_unit(kg, 0, lane, D) * 4;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll

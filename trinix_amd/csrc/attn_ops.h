@@ -169,7 +169,7 @@ struct Ops32 {
     for (int t = 0; t < DT; ++t) f.r[t] = *(const f32x4_any*)(row + t * 8 + g * 4);
     return f;
   }
-  __device__ static int swz(int u, int row) { return u ^ (row & 15); }
+  __device__ static int swz(int u, int row) { return u ^ swz_f32(row); }
 
   // The k pairs of MFMA (t, e) are d = 8t + e (lanes 0..31) and 8t + 4 + e.
   __device__ f32x16_t scores(const char* tile, const Frag& f) const {
@@ -276,8 +276,8 @@ struct TileCopy {
     for (int l = 0; l < PER; ++l) off[l] = offset(l, kTileRows - 1);
   }
   __device__ uint32_t offset(int l, int last) const {
-    const int unit = (wave * PER + l) * 64 + lane, row = unit / UPR;
-    return (uint32_t)min(row, last) * (uint32_t)ss * ESZ + (uint32_t)O::swz(unit % UPR, row) * 16u;
+    const int row = tile_copy_row(wave, PER, l, lane, UPR);
+    return tile32_offset(row, last, ss, ESZ, O::swz(((wave * PER + l) * 64 + lane) % UPR, row));
   }
   __device__ void operator()(const Store* base, int i0, int n, char* lds_tile, bool wide) const {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)lds_tile;

@@ -75,6 +75,31 @@ __host__ __device__ inline uint32_t tile_copy_offset(uint32_t row, int64_t ss, u
   return row * (uint32_t)ss * 2u + unit * 16u;
 }
 
+// The same for a tile of 32 rows of esz-byte elements (attn_ops.h TileCopy):
+// tile row `row`, read as row `last` where the tensor ends before it.
+__host__ __device__ inline uint32_t tile32_offset(int row, int last, int64_t ss, int esz, int unit) {
+  return (uint32_t)imin(row, last) * (uint32_t)ss * (uint32_t)esz + (uint32_t)unit * 16u;
+}
+// Swizzle of its fp32 rows.
+__host__ __device__ inline int swz_f32(int row) { return row & 15; }
+
+// ---- zero-padding of q, k and v (pad_heads.hip) ------------------------------
+// 16-byte unit t of the contiguous (B, S, H, upr * 8) output.
+struct PadUnit {
+  int64_t b;
+  int s, h, u;
+};
+__host__ __device__ inline PadUnit pad_unit(int64_t t, int upr, int H, int S) {
+  PadUnit p;
+  p.u = (int)(t % upr);
+  int64_t row = t / upr;
+  p.h = (int)(row % H);
+  row /= H;
+  p.s = (int)(row % S);
+  p.b = row / S;
+  return p;
+}
+
 // ---- forward (attn_fwd_mfma16) --------------------------------------------
 // Work item of workgroup `blk`: (batch, kv-head, q-head within the group,
 // row-block slot).  Each XCD owns whole KV-head groups, so the q-heads
@@ -259,6 +284,19 @@ __host__ __device__ inline KvPiece bwd_kv_piece(int blk, int groups, int per_gro
   }
   return pc;
 }
+// Key block of the `index`-th piece of a group, given the running piece counts
+// (end[k] = pieces of key blocks 0..k): the number of blocks that end at or
+// before it.  Pieces of block k: end[k] - end[k - 1]; the piece is the (index -
+// end[k - 1])-th of them.
+__host__ __device__ inline int bwd_piece_kblk(int ended, int num_kblk) { return imin(ended, num_kblk - 1); }
+// Partial sums of a piece: slot `slot` (= group * pieces per group + index)
+// holds 128 x D floats of dV (sb = 0), then of dK (1), four head_dim elements
+// of a key per lane: unit (key group kg < 4, 8-column group dq < D / 8, lane).
+__host__ __device__ inline int64_t bwd_part_base(int64_t slot, int sb, int D) { return (slot * 2 + sb) * 128 * D; }
+__host__ __device__ inline int bwd_part_unit(int kg, int dq, int lane, int D) { return (kg * (D / 8) + dq) * 64 + lane; }
+// The key (of the block's 128) and first head_dim element of a unit.
+__host__ __device__ inline int bwd_part_key(int unit, int D) { return unit / (D / 8 * 64) * 32 + (unit & 31); }
+__host__ __device__ inline int bwd_part_col(int unit, int D) { return unit / 64 % (D / 8) * 8 + ((unit & 63) >> 5) * 4; }
 // First item of piece `k` of np (items [first(k), first(k + 1)) of n).
 __host__ __device__ inline int bwd_piece_first(int n_items, int np, int k) { return (int)((int64_t)n_items * k / np); }
 

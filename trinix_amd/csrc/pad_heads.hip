@@ -25,14 +25,9 @@ __global__ __launch_bounds__(256) void pad_heads_kernel(const PadParams p) {
   const int n = blockIdx.y;
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= p.units[n]) return;
-  const int u = (int)(t % p.UPR);
-  int64_t row = t / p.UPR;
-  const int h = (int)(row % p.H[n]);
-  row /= p.H[n];
-  const int s = (int)(row % p.S[n]);
-  const int64_t b = row / p.S[n];
-  const uint16_t* x = p.x[n] + b * p.sb[n] + s * p.ss[n] + h * p.sh[n] + u * 8;
-  const int live = p.D - u * 8;  // elements of the unit that exist
+  const PadUnit pu = pad_unit(t, p.UPR, p.H[n], p.S[n]);
+  const uint16_t* x = p.x[n] + pu.b * p.sb[n] + pu.s * p.ss[n] + pu.h * p.sh[n] + pu.u * 8;
+  const int live = p.D - pu.u * 8;  // elements of the unit that exist
   u32x4_t w = {};
   if (p.vec[n]) {
     if (live > 0) w = *(const u32x4_t*)x;
