@@ -431,4 +431,6 @@ def test_narrow_and_padding_entry_points_reject_before_launch(lib):
     assert pad(x=None) == pad(out=None) == nat.TRINIX_ERR_NULL_POINTER
     assert pad(sizes=(0, 8, 1)) == pad(sizes=(1, 1 << 30, 1)) == pad(sizes=(1, 8, -1)) == nat.TRINIX_ERR_BAD_SHAPE
     assert pad(stride=(64, 8, 8, 2)) == pad(x=4097) == pad(out=8200) == nat.TRINIX_ERR_BAD_STRIDE
+    big = (1 << 29, 1 << 29, 1 << 29)  # more workgroups than a grid holds
+    assert pad(sizes=big) == nat.TRINIX_ERR_BAD_SHAPE
     assert lib.trinix_pad_heads(1, None, None, None, None, 80, 128, nat.TRINIX_BF16, None) == nat.TRINIX_ERR_NULL_POINTER

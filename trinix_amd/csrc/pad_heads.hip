@@ -58,6 +58,8 @@ extern "C" int trinix_pad_heads(int32_t n, const void* const* x, const int64_t* 
     if (!x[k] || !out[k]) return TRINIX_ERR_NULL_POINTER;
     if (sz[0] <= 0 || sz[1] <= 0 || sz[2] <= 0 || sz[0] >= (1ll << 30) || sz[1] >= (1ll << 30) || sz[2] >= (1ll << 30))
       return TRINIX_ERR_BAD_SHAPE;
+    // no more rows than a grid's units, before their product is formed
+    if (sz[0] * sz[1] > (1ll << 39) / sz[2]) return TRINIX_ERR_BAD_SHAPE;
     if (st[3] != 1 || ((uintptr_t)x[k] & 1) || ((uintptr_t)out[k] & 15)) return TRINIX_ERR_BAD_STRIDE;
     p.x[k] = (const uint16_t*)x[k];
     p.out[k] = (uint16_t*)out[k];
