@@ -381,7 +381,7 @@ def _launch_cached(key, q, k, v, rotary_cos, rotary_sin):
 # (and keep map) per call as on the full path.
 class _TrainLaunch:
     __slots__ = ("fwd", "bwd", "out_shape", "lse_shape", "dtype", "device", "align", "km_bytes", "do_stride",
-                 "dk_shape", "ws_bytes", "pieces", "pad", "do_align")
+                 "dk_shape", "ws_bytes", "pad", "do_align")
 
     def __init__(self, fwd, out_shape, lse_shape, dtype, device, align, km_bytes, dk_shape, pad, do_align):
         self.fwd = fwd                # AttnFwdArgs with null data pointers and seed
@@ -394,8 +394,7 @@ class _TrainLaunch:
         self.km_bytes = km_bytes      # dropout keep map bytes (0: none)
         self.do_stride = None         # dout strides the backward template was built for
         self.dk_shape = dk_shape      # shape of k (and of dk, dv)
-        self.ws_bytes = 0             # workspace of the backward, planned under
-        self.pieces = None            # this TRINIX_BWD_PIECES
+        self.ws_bytes = 0             # workspace of the backward
         self.pad = pad                # _Pad of q, k and v (a head_dim between the kernels'), or None
         self.do_align = do_align      # byte alignment dout needs
 
@@ -718,18 +717,34 @@ def _forward(q, k, v, attn_mask, causal, scale, dropout_p, window_size, alibi_sl
 def _launch_bwd(a, ws_bytes, device, d_out=None):
     """``trinix_attn_bwd``, with a workspace for dK/dV in pieces where the plan
     asks for one (kept alive by the allocator's stream order); with ``d_out``
-    the narrow entry point."""
+    the narrow entry point.  False, nothing launched, where the call wants a
+    larger workspace (TRINIX_BWD_PIECES changed since it was planned)."""
     lib = nat.load_library()
-    if d_out is not None:
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-        nat.check(lib.trinix_attn_bwd_narrow(ctypes.byref(a), d_out, ws.data_ptr(), ws_bytes,
-                                             current_stream_ptr(device)), "trinix_attn_bwd_narrow")
-    elif ws_bytes:
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-        nat.check(lib.trinix_attn_bwd_ws(ctypes.byref(a), ws.data_ptr(), ws_bytes, current_stream_ptr(device)),
-                  "trinix_attn_bwd_ws")
-    else:
+    if d_out is None and not ws_bytes:
         nat.check(lib.trinix_attn_bwd(ctypes.byref(a), current_stream_ptr(device)), "trinix_attn_bwd")
+        return True
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    if d_out is not None:
+        rc, what = lib.trinix_attn_bwd_narrow(ctypes.byref(a), d_out, ws.data_ptr(), ws_bytes,
+                                              current_stream_ptr(device)), "trinix_attn_bwd_narrow"
+    else:
+        rc, what = lib.trinix_attn_bwd_ws(ctypes.byref(a), ws.data_ptr(), ws_bytes,
+                                          current_stream_ptr(device)), "trinix_attn_bwd_ws"
+    if rc == nat.TRINIX_ERR_BAD_ARGUMENT and _bwd_workspace(a, d_out) > ws_bytes:
+        return False
+    nat.check(rc, what)
+    return True
+
+
+def _bwd_workspace(a, d_out=None):
+    """Bytes of workspace that the backward of ``a`` takes now."""
+    lib, n = nat.load_library(), ctypes.c_int64(0)
+    if d_out is not None:
+        nat.check(lib.trinix_attn_bwd_narrow_workspace(ctypes.byref(a), d_out, ctypes.byref(n)),
+                  "trinix_attn_bwd_narrow_workspace")
+    else:
+        nat.check(lib.trinix_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(n)), "trinix_attn_bwd_workspace")
+    return n.value
 
 
 def _backward(state, dout):
@@ -771,21 +786,16 @@ def _backward(state, dout):
         a.dropout_state = state["dropout_state"].data_ptr()
     if state["keep_map"] is not None:
         a.dropout_keep_map = state["keep_map"].data_ptr()
-    wsb = ctypes.c_int64(0)
-    if state["narrow"]:
-        nat.check(nat.load_library().trinix_attn_bwd_narrow_workspace(ctypes.byref(a), D, ctypes.byref(wsb)),
-                  "trinix_attn_bwd_narrow_workspace")
-    else:
-        nat.check(nat.load_library().trinix_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(wsb)),
-                  "trinix_attn_bwd_workspace")
-    _launch_bwd(a, wsb.value, qk.device, D if state["narrow"] else None)
+    narrow = D if state["narrow"] else None
+    ws_bytes = _bwd_workspace(a, narrow)
+    _launch_bwd(a, ws_bytes, qk.device, narrow)
     if ent is not None and ent.bwd is None and do is dout and state["dropout_state"] is None:
         tpl = nat.AttnBwdArgs.from_buffer_copy(a)
         tpl.q = tpl.k = tpl.v = tpl.out = tpl.dout = tpl.lse = tpl.delta = tpl.dq = tpl.dk = tpl.dv = None
         tpl.dropout_keep_map = None
         tpl.dropout_seed = 0
         ent.do_stride = tuple(do.stride())
-        ent.ws_bytes, ent.pieces = wsb.value, os.environ.get("TRINIX_BWD_PIECES")
+        ent.ws_bytes = ws_bytes
         ent.bwd = tpl
     if d_out != D:
         dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
@@ -794,9 +804,8 @@ def _backward(state, dout):
 
 def _backward_cached(state, ent, dout):
     """(dq, dk, dv) through the layout's backward template, or None when
-    dout is not laid out as the template's or the plan's switch changed."""
-    if (dout.dtype != ent.dtype or dout.stride() != ent.do_stride or dout.data_ptr() % ent.do_align
-            or os.environ.get("TRINIX_BWD_PIECES") != ent.pieces):
+    dout is not laid out as the template's or the plan no longer fits its workspace."""
+    if dout.dtype != ent.dtype or dout.stride() != ent.do_stride or dout.data_ptr() % ent.do_align:
         return None
     dev = ent.device
     a = nat.AttnBwdArgs.from_buffer_copy(ent.bwd)
@@ -811,7 +820,8 @@ def _backward_cached(state, ent, dout):
         a.dropout_seed = state["dropout"][1]
         if state["keep_map"] is not None:
             a.dropout_keep_map = state["keep_map"].data_ptr()
-    _launch_bwd(a, ent.ws_bytes, dev, None if ent.pad is None else ent.pad.head_dim)
+    if not _launch_bwd(a, ent.ws_bytes, dev, None if ent.pad is None else ent.pad.head_dim):
+        return None
     return dq, dk, dv
 
 
